@@ -39,7 +39,12 @@ void launch_gather(const Phys &, const Dev &, const Fluid<Real> &, double *, dou
 void launch_step_begin(const Phys &, const Dev &, hipStream_t, bool clear_lists = false);
 void launch_colloid(const Phys &, const Dev &, unsigned, hipStream_t);
 void launch_colloid_update(const Phys &, const Dev &, unsigned, const int2 *, int, hipStream_t);
-void launch_md_candidates(const Phys &, const Dev &, const int2 *, int, hipStream_t);
+void launch_md_candidates(const Phys &, const Dev &, const int2 *, int, bool link, hipStream_t);
+template <class Real> void launch_classify(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);
+// groups.hip
+template <class Real>
+void launch_groups(const Phys &, const Dev &, const Fluid<Real> &, HotPart<Real> *, bool final, hipStream_t);
+void launch_pair_lists(const Phys &, const Dev &, const int2 *, int, hipStream_t);
 void launch_tile_colloids(const Phys &, const Dev &, hipStream_t, bool cleared = false);
 void launch_debug_geometry(int n, const double *a, double L, const int *ia, int Li, int b, double *img_out,
                            double *mod_out, int *wrap_out, int *div_out, hipStream_t st);
@@ -124,7 +129,16 @@ struct bw_ctx {
     bool moments_ok = false;        // every replica has an even edge and even tile edges
     bw_mlp *mlp = nullptr;          // attached surrogate network
     MlpBuf mbuf;                    // its activations for the step's inference
-    hipGraphExec_t graphs[2][2][2] = {};  // [cur][cb][final]
+    hipGraphExec_t graphs[2][2][2][2] = {};  // [cur][cb][final][by groups]
+    // colloid groups: the step may run by groups; working copies of their
+    // particles; what k_groups_redo had to take (host memory that the device
+    // writes), what of it has been looked at and after how many steps, and the
+    // steps still to run per substep because of it
+    bool groups = false;
+    HotPart<float> *hot32 = nullptr;
+    HotPart<double> *hot64 = nullptr;
+    int *redo_stat = nullptr;
+    int redo_seen = 0, group_steps = 0, skip_groups = 0;
 };
 
 namespace {
@@ -284,13 +298,11 @@ int sync_injected(bw_ctx *c) {
 }
 
 void destroy_graphs(bw_ctx *c) {
-    for (int a = 0; a < 2; a++)
-        for (int b = 0; b < 2; b++)
-            for (int k = 0; k < 2; k++)
-                if (c->graphs[a][b][k]) {
-                    hipGraphExecDestroy(c->graphs[a][b][k]);
-                    c->graphs[a][b][k] = nullptr;
-                }
+    for (hipGraphExec_t *g = &c->graphs[0][0][0][0]; g < &c->graphs[0][0][0][0] + 16; g++)
+        if (*g) {
+            hipGraphExecDestroy(*g);
+            *g = nullptr;
+        }
 }
 
 // ---------------------------------------------------------------- the step
@@ -300,6 +312,12 @@ template <>
 Fluid<float> &fluid_of<float>(bw_ctx *c, int buf) { return c->fl[buf].f32; }
 template <>
 Fluid<double> &fluid_of<double>(bw_ctx *c, int buf) { return c->fl[buf].f64; }
+template <class Real>
+HotPart<Real> *hot_of(bw_ctx *c);
+template <>
+HotPart<float> *hot_of<float>(bw_ctx *c) { return c->hot32; }
+template <>
+HotPart<double> *hot_of<double>(bw_ctx *c) { return c->hot64; }
 
 // kernel families for bw_profile_steps
 struct Prof {
@@ -319,11 +337,13 @@ struct Prof {
 // Entry state: the run() colloid kick, old_force copy and first update_pos_md
 // of this step done (by the previous step's last colloid update or the
 // prologue).  `final`: the last colloid update stops after
-// update_velocity_colloid.
+// update_velocity_colloid.  groups: the substeps by colloid groups (same
+// results) instead of kernel by kernel over all colloids.
 template <class Real>
-int enqueue_step(bw_ctx *c, int cur, int cb, bool final, Prof *prof) {
+int enqueue_step(bw_ctx *c, int cur, int cb, bool final, bool groups, Prof *prof) {
     hipStream_t st = c->st;
-    const Phys &ph = c->ph;
+    Phys ph = c->ph;
+    ph.groups = groups;
     const bool col = c->nc_total > 0;
     Fluid<Real> &src = fluid_of<Real>(c, cur), &dst = fluid_of<Real>(c, 1 - cur);
     Dev d0 = dev_at(c, cur, cb);
@@ -339,7 +359,7 @@ int enqueue_step(bw_ctx *c, int cur, int cb, bool final, Prof *prof) {
     }
     launch_step_begin(ph, d0, st, col);  // with colloids it also clears the tile lists
     if (col) {
-        launch_md_candidates(ph, d0, c->wgt, c->nwg, st);
+        launch_md_candidates(ph, d0, c->wgt, c->nwg, groups, st);
         launch_tile_colloids(ph, d0, st, true);
     }
     if (prof) prof->mark(st, BW_KERNEL_COLLOID);
@@ -348,6 +368,17 @@ int enqueue_step(bw_ctx *c, int cur, int cb, bool final, Prof *prof) {
     launch_srd<Real>(ph, d0, src, dst, col, false, c->block, c->srd_lds + (ph.surrogate ? srd_sur_lds() : 0), st);
     if (prof) prof->mark(st, BW_KERNEL_SRD);
     if (col && ph.surrogate) launch_sur_shell_kick<Real>(ph, dev_at(c, 1 - cur, cb), dst, st);
+    if (groups) {
+        Dev d1 = dev_at(c, 1 - cur, cb);
+        launch_classify<Real>(ph, d1, dst, st);
+        if (prof) prof->mark(st, BW_KERNEL_STREAM);
+        launch_groups<Real>(ph, d1, dst, hot_of<Real>(c), final, st);
+        if (prof) prof->mark(st, BW_KERNEL_COLLIDE);
+        cb = 1 - cb;
+        if (final) launch_pair_lists(ph, dev_at(c, 1 - cur, cb), c->wgt, c->nwg, st);
+        if (prof) prof->mark(st, BW_KERNEL_COLLOID);
+        return cb;
+    }
     for (int l = 0; l < ph.n_sub; l++) {
         Dev d1 = dev_at(c, 1 - cur, cb);
         // blocked without colloids: the rotation pass did all the streaming
@@ -376,19 +407,40 @@ void enqueue_prologue(bw_ctx *c) {
 }
 
 template <class Real>
-int build_graph(bw_ctx *c, int cur, int cb, int final) {
+int build_graph(bw_ctx *c, int cur, int cb, int final, int groups) {
     hipGraph_t g;
     HIPCHK(c, hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-    enqueue_step<Real>(c, cur, cb, final != 0, nullptr);
+    enqueue_step<Real>(c, cur, cb, final != 0, groups != 0, nullptr);
     HIPCHK(c, hipStreamEndCapture(c->st, &g));
-    HIPCHK(c, hipGraphInstantiate(&c->graphs[cur][cb][final], g, nullptr, nullptr, 0));
+    HIPCHK(c, hipGraphInstantiate(&c->graphs[cur][cb][final][groups], g, nullptr, nullptr, 0));
     hipGraphDestroy(g);
     return BW_OK;
 }
 
-// colloid buffer after one step from buffer cb: one flip per update_pos_md
-int cb_after(const bw_ctx *c, int cb, bool final) {
+// Whether the next step runs by groups.  What k_groups_redo takes is slow there
+// (its one workgroup needs about half of what the per-substep launches of a
+// whole step need, more with many colloids): where more than a third of the
+// steps redid some, or one redid far more colloids than a group holds, the next
+// steps run per substep, with the same results.
+bool by_groups(bw_ctx *c) {
+    if (!c->groups) return false;
+    volatile int *redone = c->redo_stat;
+    if (c->skip_groups == 0 && (++c->group_steps >= 20 || redone[1] > 2 * GROUP_MAX)) {
+        if (redone[0] - c->redo_seen > c->group_steps / 3 || redone[1] > 2 * GROUP_MAX) c->skip_groups = 200;
+        c->redo_seen = redone[0];
+        redone[1] = 0;
+        c->group_steps = 0;
+    }
+    if (c->skip_groups == 0) return true;
+    c->skip_groups--;
+    return false;
+}
+
+// colloid buffer after one step from buffer cb: one flip per update_pos_md,
+// or one in all by groups
+int cb_after(const bw_ctx *c, int cb, bool final, bool groups) {
     if (c->nc_total == 0) return cb;
+    if (groups) return cb ^ 1;
     int npos = c->ph.n_sub - 1 + (final ? 0 : 1);
     return cb ^ (npos & 1);
 }
@@ -402,10 +454,11 @@ int do_steps(bw_ctx *c, int n) {
     c->pending_prologue = false;
     for (int s = 0; s < n; s++) {
         int fin = (s == n - 1) ? 1 : 0;
-        if (!c->graphs[c->cur][c->cb][fin])
-            if ((rc = build_graph<Real>(c, c->cur, c->cb, fin))) return rc;
-        HIPCHK(c, hipGraphLaunch(c->graphs[c->cur][c->cb][fin], c->st));
-        c->cb = cb_after(c, c->cb, fin != 0);
+        const int grp = by_groups(c) ? 1 : 0;
+        if (!c->graphs[c->cur][c->cb][fin][grp])
+            if ((rc = build_graph<Real>(c, c->cur, c->cb, fin, grp))) return rc;
+        HIPCHK(c, hipGraphLaunch(c->graphs[c->cur][c->cb][fin][grp], c->st));
+        c->cb = cb_after(c, c->cb, fin != 0, grp != 0);
         c->cur ^= 1;
         c->steps_done++;
     }
@@ -423,7 +476,7 @@ int do_profile(bw_ctx *c, int n, double *ms, int *launches) {
     for (int s = 0; s < n; s++) {
         if (c->pending_prologue) enqueue_prologue<Real>(c);
         c->pending_prologue = false;
-        c->cb = enqueue_step<Real>(c, c->cur, c->cb, s == n - 1, &prof);
+        c->cb = enqueue_step<Real>(c, c->cur, c->cb, s == n - 1, by_groups(c), &prof);
         c->cur ^= 1;
         c->steps_done++;
     }
@@ -443,6 +496,58 @@ int do_profile(bw_ctx *c, int n, double *ms, int *launches) {
 }
 
 // ------------------------------------------------------------------ create
+// Whether the fused step may run by colloid groups, and its device memory.
+// Blocked streaming only; thermal reflections must stay within the groups'
+// clearance (8 thermal speeds, beyond which a particle's draw has a chance of
+// 1e-13), and groups must stay small: in replicas of more colloids than a group
+// holds, fewer than 0.8 others within the linking distance on average (the
+// clusters of overlapping spheres become unbounded at about 2.7).
+int setup_groups(bw_ctx *c) {
+    Phys &ph = c->ph;
+    Dev &d = c->dv;
+    if (!c->block || c->nc_total == 0) return BW_OK;
+    if (8.0 * ph.vscale_thermal * ph.ndt > ph.group_reach) return BW_OK;
+    double density = 0;
+    for (const auto &R : c->reps) {
+        density = std::max(density, (double)R.p.density);
+        const double link = sqrt(ph.link2);
+        if (R.nc > GROUP_MAX && R.nc / ((double)R.L * R.L * R.L) * 4.19 * link * link * link > 0.8 + 4.19 * pow(ph.sigma, 3) * R.nc / ((double)R.L * R.L * R.L))
+            return BW_OK;
+    }
+    // a bucket holds a ball of the farthest reach around a colloid, filled (a
+    // state uploaded with particles inside colloids), with a quarter to spare
+    const double ball = 4.19 * pow(0.5 * ph.sigma + ph.margin + ph.group_reach, 3) * density;
+    const long long cap = ((long long)(1.25 * ball) + 64 + 63) / 64 * 64;
+    if (cap * c->nc_total > c->total_slots) return BW_OK;
+    const size_t NC = c->nc_total, NH = NC * (size_t)cap;
+    d.hot_cap = (int)cap;
+    // windows: about 50 selected particles per wave, from the shell that
+    // particles (mean speed 1.6 thermal) and a colloid (1.6, and tight0) cross
+    // per substep
+    const double area = 3.1416 * ph.sigma * ph.sigma, vc = sqrt(ph.kbt / ph.mass_colloid);
+    const double sel = density * area * ph.dt * (1.6 * ph.vscale_thermal + 5.8 * vc);
+    ph.window = (int)std::max(1.0, std::min((double)ph.n_sub, 50.0 / sel));
+    ph.window_min = std::max(1, ph.window / 3);
+    // a colloid's events per substep must fit a group's list with room to spare
+    if (density * area * 0.4 * ph.vscale_thermal * ph.dt > 12.0) return BW_OK;
+    int rc;
+    if ((rc = dalloc(c, &d.uf, NC)) || (rc = dalloc(c, &d.uf_linked, NC)) || (rc = dalloc(c, &d.grp_root, 4 * NC)) ||
+        (rc = dalloc(c, &d.grp_hot, NC)) || (rc = dalloc(c, &d.grp_slot, NH)) ||
+        (rc = dalloc(c, &d.grp_mem, NC)) || (rc = dalloc(c, &d.grp_big, NC)) || (rc = dalloc(c, &d.grp_small, NC)) ||
+        (rc = dalloc(c, &d.grp_cnt, 2)) || (rc = dalloc(c, &d.hot_cnt, NC)) ||
+        (rc = dalloc(c, &d.hot_ent, NH)) || (rc = dalloc(c, &d.ovl_cnt, 1)) || (rc = dalloc(c, &d.ovl_g, OVL_CAP)) ||
+        (rc = dalloc(c, &d.ovl_slot, OVL_CAP)) || (rc = dalloc(c, &d.redo, NC)) || (rc = dalloc(c, &d.redo_list, NC)) ||
+        (rc = dalloc(c, &d.redo_cnt, c->n_rep)) ||
+        (rc = dalloc(c, &d.redo_mark, 3)))
+        return rc;
+    if ((rc = c->fp64 ? dalloc(c, &c->hot64, NH) : dalloc(c, &c->hot32, NH))) return rc;
+    HIPCHK(c, hipHostMalloc((void **)&c->redo_stat, 2 * sizeof(int), hipHostMallocMapped));
+    c->redo_stat[0] = c->redo_stat[1] = 0;
+    HIPCHK(c, hipHostGetDevicePointer((void **)&d.redo_stat, c->redo_stat, 0));
+    c->groups = true;
+    return BW_OK;
+}
+
 int create_impl(const bw_params *ps, int n_rep, bw_ctx **out) {
     *out = nullptr;
     if (!ps || n_rep < 1) return BW_ERR_ARG;
@@ -499,6 +604,17 @@ int create_impl(const bw_params *ps, int n_rep, bw_ctx **out) {
     ph.near_reach = (int)floor(ph.near_base + ph.vcap_ndt) + 1;
     c->block = p0.streaming == BW_STREAM_BLOCKED && ph.near_reach <= TILE_LIST_REACH_HOST - 1;
     ph.n_rep = n_rep;
+    // groups: colloids that pair forces (the cutoff) or a reflected particle
+    // (its surface to the next, 0.9 cells of travel) can connect within the
+    // step, each colloid within `margin` of its start
+    ph.group_reach = 0.9;
+    {
+        const double link = std::max(ph.r_cutoff, p0.sigma + ph.group_reach) + 2 * ph.margin;
+        ph.link2 = link * link;
+    }
+    // 4.2 thermal flights: the collisions of a step change a colloid's
+    // displacement in it by a fraction of one
+    ph.tight0 = 4.2 * sqrt(p0.kbt / p0.mass_colloid) * p0.ndt;
     // replicas
     int cap = 0;
     long long tiles = 0, cells = 0, nf = 0;
@@ -689,6 +805,7 @@ int create_impl(const bw_params *ps, int n_rep, bw_ctx **out) {
     c->nwg = (int)wgt.size();
     if ((rc = dalloc(c, &c->wgt, std::max<size_t>(wgt.size(), 1)))) { *out = c; return rc; }
     if (!wgt.empty()) hipMemcpy(c->wgt, wgt.data(), sizeof(int2) * wgt.size(), hipMemcpyHostToDevice);
+    if ((rc = setup_groups(c))) { *out = c; return rc; }
     // injected-draw buffers exist (empty) from the start
     c->inj_dirty = ph.draws == BW_DRAWS_INJECTED;
     if ((rc = sync_injected(c))) { *out = c; return rc; }
@@ -860,6 +977,7 @@ BW_API int bw_ctx_destroy(bw_ctx *c) {
     if (c->st) hipStreamSynchronize(c->st);
     destroy_graphs(c);
     for (void *q : c->allocs) hipFree(q);
+    if (c->redo_stat) hipHostFree(c->redo_stat);
     mlp_buf_free(c->mbuf);
     const void *inj[] = {c->dv.inj_shift, c->dv.inj_axes, c->dv.inj_off, c->dv.inj_pid, c->dv.inj_val,
                          c->dv.sur_lo, c->dv.sur_hi};
@@ -1069,7 +1187,7 @@ BW_API int neighbour_list_md(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
     if (c->nc_total == 0) return BW_OK;
     Dev d = dev_for(c, c->cur);
-    launch_md_candidates(c->ph, d, c->wgt, c->nwg, c->st);
+    launch_md_candidates(c->ph, d, c->wgt, c->nwg, false, c->st);
     launch_colloid(c->ph, d, PH_MDLIST, c->st);
     return BW_OK;
 }

@@ -11,6 +11,8 @@
 #pragma once
 #include <stdint.h>
 
+#include <hip/hip_vector_types.h>
+
 #include <algorithm>
 
 namespace bw {
@@ -38,6 +40,10 @@ constexpr double MD_SKIN = 2.0;     // candidate-list skin for the colloid pair 
 constexpr double STREAM_MARGIN = 0.25;  // colloid displacement bound within a step (blocked streaming)
 constexpr int N_FEAT = 144;         // surrogate features per colloid
 constexpr int COARSE_MAX = 64;      // coarse cells of one tile
+constexpr int GROUP_SMALL = 1;      // colloids of a group that one wave of k_groups takes
+constexpr int GROUP_MAX = 24;       // colloids of a group that a workgroup of it takes
+constexpr int GROUP_LDS_COLLOIDS = 3072;  // colloids that k_group_lists holds in LDS
+constexpr int OVL_CAP = 65536;      // hot particles beyond a full bucket, all colloids
 constexpr long long MEAN_CHUNK = 65536;  // particles per workgroup of the start-up's mean
 // workgroups per replica of the start-up's mean for replicas of up to max_nf particles
 inline int init_mean_chunks(long long max_nf) { return (int)std::max(1LL, (max_nf + MEAN_CHUNK - 1) / MEAN_CHUNK); }
@@ -74,6 +80,15 @@ struct Phys {
     // position at the step's start
     double margin, near_base, near_shell2, vcap_ndt;
     int near_reach;                   // per-axis cell reach of the near test
+    // colloid groups (fused step): colloids closer than sqrt(link2) at the
+    // step's start share a group; a reflected particle that travels less than
+    // group_reach stays clear of every other group; tight0 is the thermal part
+    // of the bound on a colloid's displacement in a step by which a group's
+    // windows (`window` substeps for one colloid and wave, at least window_min)
+    // are laid out
+    double link2, group_reach, tight0;
+    int window, window_min;
+    int groups;                       // the step runs by groups
     int moments;                      // SRD pass writes coarse-cell moments (surrogate inputs)
     int surrogate;                    // colloids may be driven by the surrogate impulses
     int n_sub;
@@ -81,6 +96,7 @@ struct Phys {
     int srd_threads;                  // SRD workgroup size
     int srd_pt;                       // SRD slots per thread (srd_threads x srd_pt >= cap)
     int near_blocks;                  // grid of the near-particle pass
+    int classify_blocks;              // grid of the grouped step's classification
     int near_wrap;                    // the SRD near test needs the periodic wrap (a small box)
     int n_rep, n_tiles, n_colloid_total;
     int draws;                        // BW_DRAWS_*
@@ -103,6 +119,15 @@ struct Fluid {
     Real *ox, *oy, *oz;
     Real *vx, *vy, *vz;
     int *pid;
+};
+
+// Working copy of a particle that may reach a colloid, group by group
+template <class Real>
+struct alignas(8) HotPart {
+    Real ox, oy, oz;
+    int cell;
+    Real vx, vy, vz;
+    int pid;
 };
 
 struct Dev {
@@ -131,6 +156,23 @@ struct Dev {
     int *cont_cnt, *cont_slot, *cont_from;  // continuations of the colloid loop
     double *cont_dump;
     int *ovf_cnt, *ovf_list, *ev_total;     // per replica: overflowed buckets, events seen
+    // colloid groups (fused step)
+    int *uf;             // per colloid: parent in its group's tree (the root is the group's first colloid)
+    int *uf_linked;      // per colloid: its group has other colloids
+    int *grp_root;       // k_group_lists' arrays (4 per colloid) where LDS does not hold them
+    int *grp_mem;        // the members, group by group
+    int *grp_hot;        // per root: the group's place among the working copies and slots
+    int *grp_slot;       // the working copies' slots
+    int2 *grp_big, *grp_small;  // groups of more than / up to GROUP_SMALL colloids: first member, size
+    int *grp_cnt;        // their numbers
+    int *hot_cnt, *hot_ent;  // per colloid: slots of the particles that may reach it in the step
+    int hot_cap;
+    int *ovl_cnt, *ovl_g, *ovl_slot;  // entries beyond a full bucket
+    int *redo;           // per colloid: its group is left to k_groups_redo
+    int *redo_list;      // per replica (at its first colloid): those colloids
+    int *redo_cnt;       // per replica
+    int *redo_mark;      // the last step that redid any, the number of such steps, the most colloids in one
+    int *redo_stat;      // the last two in host memory
     unsigned *status;
     long long *step;     // MPCD step counter (device generator key)
     double *shift;       // [n_rep*3] shift of the current step

@@ -141,7 +141,12 @@ __device__ __forceinline__ double img1(double a, double L) {
     return a - L * round(a / L);
 }
 // mod(a,b) = a - b*round((a - b/2)/b) (cpp/parameters.hpp:75)
-__device__ __forceinline__ double mod1(double a, double L) { return a - L * round((a - L / 2) / L); }
+// Without the division well inside the box, where the rounding gives 0 (a - 0
+// is a).  Bit-identical to the formula.
+__device__ __forceinline__ double mod1(double a, double L) {
+    if (a > 1e-3 * L && a < 0.999 * L) return a;
+    return a - L * round((a - L / 2) / L);
+}
 
 constexpr int CELL_MASK = (1 << CELL_BITS) - 1;
 // bit 30 of the packed cell: the particle is inside a colloid that was a
@@ -231,6 +236,25 @@ __device__ __forceinline__ void normalise(int &i, Real &o, int L) {
         }
     }
 }
+// normalise without branches (but for a particle that crosses several box
+// lengths): more instructions than the branches skip, but no waits for them,
+// where a wave is alone on its SIMD
+template <class Real>
+__device__ __forceinline__ void normalise_flat(int &i, Real &o, int L) {
+    const Real f = floor(o);
+    Real q = f != Real(0) ? o - f : o;  // (an offset of -0 stays as it is)
+    const bool up = q >= Real(1);
+    q = up ? Real(0) : q;
+    int j = i + (int)f + (up ? 1 : 0);
+    j = j >= L ? j - L : j;
+    j = j < 0 ? j + L : j;
+    if ((unsigned)j >= (unsigned)L) {
+        j %= L;
+        if (j < 0) j += L;
+    }
+    i = j;
+    o = q;
+}
 
 // o in [0,1) (+0 included, -0 and NaN excluded) with one integer compare
 // normalise() for a particle that moves less than one cell in all: the cell
@@ -267,6 +291,26 @@ __device__ __forceinline__ bool in_unit3(double a, double b, double c) {
             (unsigned long long)__double_as_longlong(c)) < 0x3FF0000000000000ull;
 }
 
+
+// one particle streamed through n substeps (cpp/update.cpp:56-60); FLAT: by
+// normalise_flat
+template <bool FLAT, class Real>
+__device__ __forceinline__ void fly(int n, Real dt, int L, Real vx, Real vy, Real vz, int &ix, int &iy, int &iz,
+                                    Real &ox, Real &oy, Real &oz) {
+    const Real dx = vx * dt, dy = vy * dt, dz = vz * dt;
+    auto norm = [&](int &i, Real &o) {
+        if constexpr (FLAT) normalise_flat(i, o, L);
+        else normalise(i, o, L);
+    };
+    for (int l = 0; l < n; l++) {
+        ox = ox + dx;
+        oy = oy + dy;
+        oz = oz + dz;
+        norm(ix, ox);
+        norm(iy, oy);
+        norm(iz, oz);
+    }
+}
 
 // ------------------------------------------------------------ reflection
 // Stochastic (thermal-wall) reflection, cpp/fluid_colloid_collision.cpp:7-24:
@@ -344,6 +388,39 @@ __device__ __forceinline__ bool near_interval(int c, int lo, int len, int L) {
     return wrapi(c - lo, L) < len;
 }
 
+// the cell is farther than TILE_REACH from the tile that owns the slot
+__device__ inline bool outside_tile_reach(const Rep &R, int cap, int slot, int ix, int iy, int iz) {
+    const int lt = slot / cap - R.first_tile;
+    const int tx = lt % R.nt[0], ty = (lt / R.nt[0]) % R.nt[1], tz = lt / (R.nt[0] * R.nt[1]);
+    return !(near_interval(ix, tx * R.B[0] - TILE_REACH, R.B[0] + 2 * TILE_REACH, R.L) &&
+             near_interval(iy, ty * R.B[1] - TILE_REACH, R.B[1] + 2 * TILE_REACH, R.L) &&
+             near_interval(iz, tz * R.B[2] - TILE_REACH, R.B[2] + 2 * TILE_REACH, R.L));
+}
+
+// ------------------------------------------------------------ colloid groups
+// The colloids of a replica in groups that cannot act on each other within a
+// step: a tree per group in uf (each parent has a lower index, so the root is
+// the group's first colloid), built with atomics by the pair-candidate pass
+// (colloids near each other) and the classification (colloids that one
+// particle may reach both).
+__device__ __forceinline__ int group_parent(const Dev &d, int g) {
+    return __hip_atomic_load(&d.uf[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline int group_find(const Dev &d, int g) {
+    for (int p = group_parent(d, g); p != g; p = group_parent(d, g)) g = p;
+    return g;
+}
+__device__ inline void group_join(const Dev &d, int a, int b) {
+    d.uf_linked[a] = 1;
+    d.uf_linked[b] = 1;
+    for (;;) {
+        a = group_find(d, a);
+        b = group_find(d, b);
+        if (a == b) return;
+        if (a < b) { const int t = a; a = b; b = t; }
+        if (atomicCAS(&d.uf[a], a, b) == a) return;  // a was a root: now below b < a
+    }
+}
 // Colloids that can touch a particle of a tile during one MPCD step: a
 // particle stays within TILE_REACH cells of its tile box, the collision and
 // run() stencils reach 3 cells and a colloid's cell moves by at most one cell
@@ -726,14 +803,15 @@ struct ShellPay {
     double u[3], a[3];
     bool lin, ang;
 };
-__device__ inline ShellPay shell_pay(const Phys &ph, const Dev &d, int g) {
+// ra: the colloid's orientation
+__device__ inline ShellPay shell_pay(const Phys &ph, const Dev &d, int g, const double *ra) {
     ShellPay p;
     const int cnt = d.sshell[g];
     const unsigned long long *q = d.sacc + (size_t)SUR_ACC * g;
     const double ratio = ph.mass_colloid / ph.mass_fl, v0 = d.cv0[g], ns = (double)ph.n_sub;
     double D[3], A[3], s1[3];
     for (int k = 0; k < 3; k++) {
-        D[k] = (ns * d.csur[6 * g + k] + unfixq(q[k])) + ratio * (d.cra[3 * g + k] * v0);
+        D[k] = (ns * d.csur[6 * g + k] + unfixq(q[k])) + ratio * (ra[k] * v0);
         A[k] = ns * d.csur[6 * g + 3 + k] + unfixq(q[3 + k]);
         s1[k] = unfixq(q[6 + k]);
         p.u[k] = 0.0;
@@ -808,7 +886,7 @@ __device__ inline void colloid_load(const Phys &ph, const Dev &d, int g, unsigne
     // fluid) or its torque (no invertible inertia) takes the mirrored fluid's
     // momentum or angular momentum change back instead
     if (in.sur) {
-        const ShellPay pay = shell_pay(ph, d, g);
+        const ShellPay pay = shell_pay(ph, d, g, d.cra + 3 * g);
         const unsigned long long *q = d.sacc + (size_t)SUR_ACC * g;
         for (int k = 0; k < 3; k++) {
             if (!pay.lin) in.sv[k] = -unfixq(q[k]) / ph.n_sub;

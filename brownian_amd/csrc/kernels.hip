@@ -16,6 +16,7 @@
 //             k_colloid_update  1 wave / colloid: collision impulse, activity,
 //                                WCA force, velocity, [kick], position }
 #include "bw_device.h"
+#include "collide.h"
 
 namespace bw {
 
@@ -30,6 +31,12 @@ __global__ void k_step_begin(Phys ph, Dev d, int clear_lists) {
         }
         for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < ph.n_rep; r += gridDim.x * blockDim.x)
             d.tcl_stale[r] = 0;
+        if (ph.groups)  // every colloid its own group, with no particles
+            for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < ph.n_colloid_total; g += gridDim.x * blockDim.x) {
+                d.uf[g] = g;
+                d.uf_linked[g] = 0;
+                d.hot_cnt[g] = 0;
+            }
     }
     if (blockIdx.x != 0) return;
     long long s = *d.step + 1;
@@ -50,6 +57,7 @@ __global__ void k_step_begin(Phys ph, Dev d, int clear_lists) {
     if (threadIdx.x == 0) {
         *d.step = s;
         *d.chunk_cnt = 0;
+        if (ph.groups) *d.ovl_cnt = 0;
     }
 }
 
@@ -61,7 +69,8 @@ __global__ void k_colloid(Phys ph, Dev d, unsigned flags) {
 }
 
 // one wave per colloid: every partner within cutoff + skin, ascending
-__global__ __launch_bounds__(256) void k_md_candidates(Phys ph, Dev d, const int2 *wgt) {
+// link: also joins the groups of colloids closer than sqrt(link2)
+__global__ __launch_bounds__(256) void k_md_candidates(Phys ph, Dev d, const int2 *wgt, int link) {
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int2 wt = wgt[blockIdx.x];
     const Rep R = d.rep[wt.x];
@@ -87,7 +96,9 @@ __global__ __launch_bounds__(256) void k_md_candidates(Phys ph, Dev d, const int
             bool p = false;
             if (m < R.nc && j != g) {
                 double tx = img1(pi[0] - pj[u][0], L), ty = img1(pi[1] - pj[u][1], L), tz = img1(pi[2] - pj[u][2], L);
-                p = (tx * tx + ty * ty) + tz * tz < ph.lim_md_skin;
+                const double r2 = (tx * tx + ty * ty) + tz * tz;
+                p = r2 < ph.lim_md_skin;
+                if (link && j < g && r2 < ph.link2) group_join(d, g, j);
             }
             unsigned long long b = __ballot(p);
             int rank = __popcll(b & ((1ull << lane) - 1ull));
@@ -1251,7 +1262,7 @@ struct StreamOp {
     __device__ __forceinline__ unsigned all_listed() const {
         return tc.n >= MASK_BITS ? 0xffffffffu : ((1u << tc.n) - 1u);
     }
-    __device__ __forceinline__ void operator()(int slot, int c, Real ox, Real oy, Real oz, Real vx, Real vy, Real vz) {
+    __device__ __forceinline__ void operator()(int slot, int c, Real ox, Real oy, Real oz, Real &vx, Real &vy, Real &vz) {
         int ix, iy, iz;
         unpack_cell(c, ix, iy, iz);
         const int phantom = c & PHANTOM;
@@ -1470,430 +1481,142 @@ __global__ __launch_bounds__(256, KICK ? 1 : 8) void k_stream_near(Phys ph, Dev 
     if (ch_over) atomicOr(d.status, BW_FLAG_CHAIN_OVERFLOW);
 }
 
-// --------------------------------------------------------------- collisions
-// One event: back half-step, stochastic reflection with the colloid's rigid
-// body velocity, forward half-step (cpp/fluid_colloid_collision.cpp:36-43).
-// (bx,by,bz) is the offset in the binned cell (ix,iy,iz), updated in place.
-__device__ inline void reflect_event(const Phys &ph, int L, int ix, int iy, int iz, double &bx, double &by,
-                                     double &bz, double &vx, double &vy, double &vz, const double *pc,
-                                     const double *vcol, const double *wcol, const ReflDraw &dr, double *rs,
-                                     bool fp32) {
-    const double Ld = (double)L, dt = ph.dt;
-    bx = bx - vx * dt * 0.5;
-    by = by - vy * dt * 0.5;
-    bz = bz - vz * dt * 0.5;
-    double ax = (double)ix + bx, ay = (double)iy + by, az = (double)iz + bz;
-    double rsx = img1(ax - pc[0], Ld), rsy = img1(ay - pc[1], Ld), rsz = img1(az - pc[2], Ld);
-    double ux, uy, uz;
-    stochastic_reflection(ph, Ld, ax, ay, az, rsx, rsy, rsz, dr, ux, uy, uz);
-    double nx = ux + vcol[0] + (wcol[1] * rsz - wcol[2] * rsy);
-    double ny = uy + vcol[1] + (wcol[2] * rsx - wcol[0] * rsz);
-    double nz = uz + vcol[2] + (wcol[0] * rsy - wcol[1] * rsx);
-    if (fp32) {  // what the velocity store keeps
-        nx = (double)(float)nx; ny = (double)(float)ny; nz = (double)(float)nz;
+// The grouped step's first pass over the near particles (chunks as in
+// k_stream_near): the run() kick, then, for each particle, the colloids it may
+// reach within the step -- closer than the radius plus its travel plus the
+// displacement bound of blocked streaming.  A particle that reaches none is
+// streamed through the whole step here; the others go to the bucket of the
+// first such colloid, whose group (k_groups) streams it, and the groups of the
+// colloids it may reach are joined.
+template <class Real>
+__global__ __launch_bounds__(256) void k_classify(Phys ph, Dev d, Fluid<Real> f) {
+    static_assert(TCL_CAP == 64, "one lane per listed colloid");
+    __shared__ TileColl s_tc[4];
+    __shared__ NearColl s_nf[4];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    TileColl &tc = s_tc[w];
+    NearColl &nf = s_nf[w];
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const int nchunk = ld_const(d.chunk_cnt);
+    const int stride = gridDim.x * 4;
+    bool drift = false;
+    int ch = blockIdx.x * 4 + w;
+    int e = ch < nchunk ? ld_const(d.chunk_tile + ch) : 0;
+    for (; ch < nchunk; ch += stride) {
+        const int T = e >> 6, i = ((e & 63) << 6) + lane;
+        if (ch + stride < nchunk) e = ld_const(d.chunk_tile + ch + stride);  // next chunk, ahead of its use
+        const int r = ld_const(d.tile_rep + T);
+        const int cnt = min(ld_const(d.tcl_cnt + T), TCL_CAP);  // the step's list: no colloid has moved since
+        const int gl = d.tcl_list[T * TCL_CAP + lane];
+        const int n = min(ld_const(d.near_cnt + T), ph.cap);
+        const int slot = T * ph.cap + i;
+        int c0 = 0;
+        Real ox = 0, oy = 0, oz = 0, vx = 0, vy = 0, vz = 0;
+        if (i < n) {
+            c0 = f.cell[slot];
+            ox = f.ox[slot]; oy = f.oy[slot]; oz = f.oz[slot];
+            vx = f.vx[slot]; vy = f.vy[slot]; vz = f.vz[slot];
+        }
+        wave_sync();  // the previous chunk's lanes are done with the LDS lists
+        const Rep R = ld_const(d.rep + r);
+        const int L = R.L;
+        const int lt = T - R.first_tile;
+        const int tx = lt % R.nt[0], ty = (lt / R.nt[0]) % R.nt[1], tz = lt / (R.nt[0] * R.nt[1]);
+        const int bx0 = tx * R.B[0], by0 = ty * R.B[1], bz0 = tz * R.B[2];
+        if (lane < cnt) {
+            load_tile_slot(d, ph, gl, lane, true, tc);
+            const double Ld = (double)L;
+            nf.cx[lane] = (float)img1(tc.px[lane] - bx0, Ld);
+            nf.cy[lane] = (float)img1(tc.py[lane] - by0, Ld);
+            nf.cz[lane] = (float)img1(tc.pz[lane] - bz0, Ld);
+            nf.rx[lane] = (float)img1(tc.rx[lane] - bx0, Ld);
+            nf.ry[lane] = (float)img1(tc.ry[lane] - by0, Ld);
+            nf.rz[lane] = (float)img1(tc.rz[lane] - bz0, Ld);
+        }
+        if (lane == 0) tc.n = cnt;
+        wave_sync();
+        const Region rg = tile_region(R, tx, ty, tz);
+        StreamOp<Real, true, false, false, TileColl, true> op{ph, d, f, tc, rg, nullptr, nullptr, L, r, 0, 0, 0, 0, 0, 0,
+                                                              false, false, &nf, bx0, by0, bz0, ph.near_wrap != 0};
+        int home = -1;
+        if (i < n) {
+            op(slot, c0, ox, oy, oz, vx, vy, vz);  // the run() kick
+            int ix, iy, iz;
+            unpack_cell(c0, ix, iy, iz);
+            const float px = (float)pdiff(ix, bx0, L) + (float)ox, py = (float)pdiff(iy, by0, L) + (float)oy,
+                        pz = (float)pdiff(iz, bz0, L) + (float)oz;
+            const float wx = (float)vx, wy = (float)vy, wz = (float)vz;
+            // 2e-2 cells cover the FP32 roundings of positions and travel
+            const float rc = sqrtf((float)ph.lim_coll) + sqrtf((wx * wx + wy * wy) + wz * wz) * (float)ph.ndt +
+                             (float)ph.margin + 0.02f;
+            const float rc2 = rc * rc;
+            for_listed(tc, [&](int k) {
+                if (op.d2f(px, py, pz, nf.cx[k], nf.cy[k], nf.cz[k]) <= rc2) {
+                    if (home < 0) home = tc.g[k];
+                    else group_join(d, home, tc.g[k]);
+                }
+            });
+            if (home < 0) {
+                // (a phantom that is inside no colloid ends being one)
+                fly<false>(ph.n_sub, (Real)ph.dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
+                f.cell[slot] = pack_cell(ix, iy, iz);
+                f.ox[slot] = ox; f.oy[slot] = oy; f.oz[slot] = oz;
+                if (outside_tile_reach(R, ph.cap, slot, ix, iy, iz)) drift = true;
+            }
+        }
+        // into the buckets: one atomic per distinct home of the wave, all of
+        // them in flight together
+        int lead = -1, rank = 0, num = 0;
+        for (unsigned long long pending = __ballot(home >= 0); pending;) {
+            const int src = __ffsll((long long)pending) - 1;
+            const unsigned long long m = __ballot(home == lane_value(home, src));
+            if (m & (1ull << lane)) {
+                lead = src;
+                rank = __popcll(m & below);
+                num = __popcll(m);
+            }
+            pending &= ~m;
+        }
+        int base = 0;
+        if (lead == lane) base = atomicAdd(&d.hot_cnt[home], num);
+        base = __shfl(base, lead < 0 ? 0 : lead);
+        if (home >= 0) {
+            if (base + rank < d.hot_cap) {
+                d.hot_ent[(size_t)home * d.hot_cap + base + rank] = slot;
+            } else {
+                const int q = atomicAdd(d.ovl_cnt, 1);
+                if (q < OVL_CAP) {
+                    d.ovl_g[q] = home;
+                    d.ovl_slot[q] = slot;
+                } else {
+                    atomicOr(d.status, BW_FLAG_LIST_OVERFLOW);
+                }
+            }
+        }
     }
-    rs[0] = rsx; rs[1] = rsy; rs[2] = rsz;
-    vx = nx; vy = ny; vz = nz;
-    bx = bx + vx * dt * 0.5;
-    by = by + vy * dt * 0.5;
-    bz = bz + vz * dt * 0.5;
+    if (drift) atomicOr(d.status, BW_FLAG_DRIFT);
 }
 
-// momentum and angular-momentum transfer of one event: dump - vel and
-// rs x (dump - vel) (cpp/fluid_colloid_collision.cpp:40-42)
-__device__ __forceinline__ void transfer(const double *dump, double vx, double vy, double vz, const double *rs,
-                                         double *c) {
-    double ex = dump[0] - vx, ey = dump[1] - vy, ez = dump[2] - vz;
-    c[0] = ex; c[1] = ey; c[2] = ez;
-    c[3] = rs[1] * ez - rs[2] * ey;
-    c[4] = rs[2] * ex - rs[0] * ez;
-    c[5] = rs[0] * ey - rs[1] * ex;
-}
-
-// One wave per colloid g: its pair list for this substep, then the particles
-// inside g and no other colloid, ranked in the reference's neigh_fl order
-// (stencil position, then id) and reflected; the momentum/torque sums are taken
-// in that order.  A particle a reflection moved into a later colloid continues
-// the reference's colloid loop serially (k_serial).  The pair partners j > g
-// (position and cell) are staged in LDS while the pair list is built, so the
-// continuation test of every event reads no global memory.
-struct PairColl {
-    double px, py, pz;
-    int cx, cy, cz;
-};
-
+// ------------------------------------------------- collisions and updates
 template <class Real>
 __global__ __launch_bounds__(COLLIDE_THREADS) void k_collide(Phys ph, Dev d, Fluid<Real> f, int substep,
                                                              const int2 *wgt) {
-    __shared__ double s_c[COLLIDE_THREADS / 64][EV_CAP][6];
-    __shared__ PairColl s_nb[COLLIDE_THREADS / 64][MD_CAP];
-    __shared__ int s_ne[COLLIDE_THREADS / 64], s_nnb[COLLIDE_THREADS / 64];
-    const bool fp32 = sizeof(Real) == 4;
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ CollideLds s[COLLIDE_THREADS / 64];
+    const int w = threadIdx.x >> 6;
     const int2 wt = ph.n_rep == 1 ? make_int2(0, blockIdx.x * (COLLIDE_THREADS / 64)) : wgt[blockIdx.x];
-    const int r = wt.x;
-    const int g = wt.y + w;
-    // Loads that do not need the replica record go first, at an in-range
-    // index (a workgroup's last colloids may lie past its replica).  Entries
-    // of the candidate list and of the event bucket past their counts are
-    // stale but valid indices, so the candidates' positions and the events'
-    // particles are requested with the counts and discarded when unused.
-    const int gs = min(g, ph.n_colloid_total - 1);
-    const int mdc_n = d.mdc_cnt[gs], ne_s = d.ev_cnt[gs];
-    const int js = d.mdc_list[gs * MDC_CAP + lane], slot_s = d.ev_slot[gs * EV_CAP + lane];
-    double pg[3], pj[3], vg[3], wg[3];
-    int cg[3], cj[3];
-    for (int k = 0; k < 3; k++) {
-        pg[k] = d.cpos[3 * gs + k];
-        pj[k] = d.cpos[3 * js + k];
-        vg[k] = d.cvel[3 * gs + k];
-        wg[k] = d.comega[3 * gs + k];
-        cg[k] = d.ccell[3 * gs + k];
-        cj[k] = d.ccell[3 * js + k];
-    }
-    const int pid_s = f.pid[slot_s], cell_s = f.cell[slot_s];
-    const Real pox_s = f.ox[slot_s], poy_s = f.oy[slot_s], poz_s = f.oz[slot_s];
-    const Real pvx_s = f.vx[slot_s], pvy_s = f.vy[slot_s], pvz_s = f.vz[slot_s];
-    const Rep R = d.rep[r];
-    const int L = R.L;
-    const double Ld = (double)L;
-    const bool valid = g < R.first_colloid + R.nc;
-    const long long step = *d.step;
-    const bool full = d.md_stale[r] != 0;
-    const int ncand = valid ? (full ? R.nc : mdc_n) : 0;
-    int ne = 0;
-    if (valid) {
-        ne = ne_s;
-        if (lane == 0) {
-            d.ev_cnt[g] = 0;
-            if (ne > EV_CAP) {
-                int k = atomicAdd(&d.ovf_cnt[r], 1);
-                if (k < OVF_CAP) d.ovf_list[r * OVF_CAP + k] = g;
-                else atomicOr(d.status, BW_FLAG_EVENT_OVERFLOW);
-            } else if (ne > 0 && ph.draws == BW_DRAWS_INJECTED) {
-                atomicAdd(&d.ev_total[r], ne);
-            }
-        }
-        if (ne > EV_CAP) ne = 0;  // full bucket: all its events are replayed serially
-    }
-    int slot = -1, pid = 0, ix = 0, iy = 0, iz = 0;
-    long long key = 0x7fffffffffffffffll;
-    Real pox = 0, poy = 0, poz = 0, pvx = 0, pvy = 0, pvz = 0;
-    if (lane < ne) {
-        slot = slot_s;
-        pid = pid_s;
-        unpack_cell(cell_s, ix, iy, iz);
-        pox = pox_s; poy = poy_s; poz = poz_s;
-        pvx = pvx_s; pvy = pvy_s; pvz = pvz_s;
-    }
-    if (valid) {  // pair list of g (cpp/neighbour_list.cpp:27-39), partners j > g into LDS
-        const unsigned long long below = (1ull << lane) - 1ull;
-        int nmd = 0, nnb = 0;
-        for (int base = 0; base < ncand; base += 64) {
-            const int m = base + lane;
-            int j = -1;
-            bool p = false;
-            const bool pre = base == 0 && !full;  // this lane's candidate is js, loaded above
-            if (m < ncand) {
-                j = pre ? js : (full ? R.first_colloid + m : d.mdc_list[g * MDC_CAP + m]);
-                p = j != g && (pre ? md_pair_at(ph, Ld, g, j, pg, pj) : md_pair(ph, d, Ld, g, j));
-            }
-            const unsigned long long b = __ballot(p);
-            const int rank = __popcll(b & below);
-            if (p && nmd + rank < MD_CAP) {
-                const int e = g * MD_CAP + nmd + rank;
-                d.md_list[e] = j;
-                // the pair's force addend, summed in list order by k_colloid_update
-                double pjv[3], t[3];
-                for (int k = 0; k < 3; k++) pjv[k] = pre ? pj[k] : d.cpos[3 * j + k];
-                force_addend(ph, Ld, g, j, pg, pjv, t);
-                for (int k = 0; k < 3; k++) d.md_f[3 * e + k] = t[k];
-            }
-            nmd += __popcll(b);
-            const bool q = p && j > g && !(ph.surrogate && d.cmode[j]);
-            const unsigned long long bq = __ballot(q);
-            const int rq = __popcll(bq & below);
-            if (q && nnb + rq < MD_CAP) {
-                PairColl &e = s_nb[w][nnb + rq];
-                if (pre) {
-                    e.px = pj[0]; e.py = pj[1]; e.pz = pj[2];
-                    e.cx = cj[0]; e.cy = cj[1]; e.cz = cj[2];
-                } else {
-                    e.px = d.cpos[3 * j]; e.py = d.cpos[3 * j + 1]; e.pz = d.cpos[3 * j + 2];
-                    e.cx = d.ccell[3 * j]; e.cy = d.ccell[3 * j + 1]; e.cz = d.ccell[3 * j + 2];
-                }
-            }
-            nnb += __popcll(bq);
-        }
-        if (lane == 0) {
-            if (nmd > MD_CAP) { atomicOr(d.status, BW_FLAG_LIST_OVERFLOW); nmd = MD_CAP; }
-            d.md_cnt[g] = nmd;
-            s_nnb[w] = min(nnb, MD_CAP);
-        }
-    }
-    wave_sync();  // the wave's pair partners and list visible to its lanes (LDS is per wave)
-    if (lane < ne) {
-        int dx = pdiff(ix, cg[0], L), dy = pdiff(iy, cg[1], L), dz = pdiff(iz, cg[2], L);
-        key = ((long long)stencil_index(dx, dy, dz) << 32) | (unsigned)pid;
-    }
-    int rank = 0;
-    for (int m = 0; m < ne; m++) {
-        long long km = lane_value(key, m);
-        rank += (km < key) ? 1 : 0;
-    }
-    if (lane < ne) {
-        double bx = pox, by = poy, bz = poz;
-        double vx = pvx, vy = pvy, vz = pvz;
-        ReflDraw dr;
-        double cont[6] = {0, 0, 0, 0, 0, 0};
-        const double dump[3] = {vx, vy, vz};
-        if (draw_reflection(d, ph, R, step, substep, g, pid, dr)) {
-            double rs[3];
-            reflect_event(ph, L, ix, iy, iz, bx, by, bz, vx, vy, vz, pg, vg, wg, dr, rs, fp32);
-            transfer(dump, vx, vy, vz, rs, cont);
-            f.ox[slot] = (Real)bx; f.oy[slot] = (Real)by; f.oz[slot] = (Real)bz;
-            f.vx[slot] = (Real)vx; f.vy[slot] = (Real)vy; f.vz[slot] = (Real)vz;
-            // The reference goes on to test this particle, now moved, against
-            // every later colloid (cpp/fluid_colloid_collision.cpp:30-35).  A
-            // later colloid that now contains it is a pair partner of g; if
-            // there is one, the rest of the colloid loop is replayed serially.
-            const double ax = (double)ix + bx, ay = (double)iy + by, az = (double)iz + bz;
-            const int nnb = s_nnb[w];
-#pragma unroll 2
-            for (int m = 0; m < nnb; m++) {
-                const PairColl &e = s_nb[w][m];
-                if (!in_stencil(ix, iy, iz, e.cx, e.cy, e.cz, L)) continue;
-                double rx = img1(e.px - ax, Ld), ry = img1(e.py - ay, Ld), rz = img1(e.pz - az, Ld);
-                if ((rx * rx + ry * ry) + rz * rz <= ph.lim_coll) {
-                    int c = atomicAdd(&d.cont_cnt[r], 1);
-                    if (c < CONT_CAP) {
-                        int q = r * CONT_CAP + c;
-                        d.cont_slot[q] = slot;
-                        d.cont_from[q] = g + 1;
-                        for (int kk = 0; kk < 3; kk++) d.cont_dump[3 * q + kk] = dump[kk];
-                    } else {
-                        atomicOr(d.status, BW_FLAG_CHAIN_OVERFLOW);
-                    }
-                    break;
-                }
-            }
-        } else {
-            atomicOr(d.status, BW_FLAG_DRAW_MISSING);
-        }
-        for (int k = 0; k < 6; k++) s_c[w][rank][k] = cont[k];
-    }
-    if (lane == 0) s_ne[w] = ne;
-    wave_sync();
-    if (lane == 0 && valid) {
-        double a[6] = {0, 0, 0, 0, 0, 0};
-#pragma unroll 2
-        for (int e = 0; e < s_ne[w]; e++)
-            for (int k = 0; k < 6; k++) a[k] = a[k] + s_c[w][e][k];
-        for (int k = 0; k < 3; k++) {
-            d.cdv[3 * g + k] = a[k];
-            d.cdw[3 * g + k] = a[3 + k];
-        }
-    }
+    collide_wave<Real>(ph, d, f, substep, wt.x, wt.y + w, s[w]);
 }
-
-// One workgroup per replica, after k_collide: the serial list -- particles
-// inside several colloids and the events of overflowed buckets (tested from
-// the replica's first colloid on, dump = current velocity), and the
-// continuations (from the colloid after the reflecting one, dump = velocity
-// before that reflection) -- replayed in ascending particle id, each particle
-// through the colloids whose stencil holds its binned cell in ascending order
-// (cpp/fluid_colloid_collision.cpp:29-49).  Then the injected-draw totals are
-// checked and the replica's counters cleared.
+// one workgroup per replica
 template <class Real>
 __global__ __launch_bounds__(COLLIDE_THREADS) void k_serial(Phys ph, Dev d, Fluid<Real> f, int substep) {
-    __shared__ int s_chain[SERIAL_CAP], s_src[SERIAL_CAP];
-    __shared__ int s_nser, s_cand_n, s_serial_events, s_inj_tot;
-    __shared__ int s_cand[TCL_CAP];
-    __shared__ int s_wt[COLLIDE_THREADS / 64];
-    const bool fp32 = sizeof(Real) == 4;
-    const int r = blockIdx.x;
-    const Rep R = d.rep[r];
-    const int L = R.L;
-    const double Ld = (double)L;
-    const int gend = R.first_colloid + R.nc;
-    const long long step = *d.step;
-    const int nchain = d.chain_cnt[r], ncont = d.cont_cnt[r], novf = min(d.ovf_cnt[r], OVF_CAP);
-    if (threadIdx.x == 0) {
-        s_serial_events = 0;
-        s_inj_tot = 0;
-        s_nser = 0;
-    }
-    __syncthreads();
-    if (nchain > 0 || ncont > 0 || novf > 0) {
-        if (threadIdx.x == 0) {
-            int n = 0;
-            int nch = min(nchain, CHAIN_CAP);
-            if (nchain > CHAIN_CAP) atomicOr(d.status, BW_FLAG_CHAIN_OVERFLOW);
-            for (int i = 0; i < nch && n < SERIAL_CAP; i++, n++) { s_chain[n] = d.chain_slot[r * CHAIN_CAP + i]; s_src[n] = -1; }
-            int nco = min(ncont, CONT_CAP);
-            if (ncont > CONT_CAP) atomicOr(d.status, BW_FLAG_CHAIN_OVERFLOW);
-            for (int i = 0; i < nco && n < SERIAL_CAP; i++, n++) { s_chain[n] = d.cont_slot[r * CONT_CAP + i]; s_src[n] = r * CONT_CAP + i; }
-            for (int i = 0; i < novf; i++) {
-                int gg = d.ovf_list[r * OVF_CAP + i];
-                for (int e = 0; e < EV_CAP && n < SERIAL_CAP; e++, n++) { s_chain[n] = d.ev_slot[gg * EV_CAP + e]; s_src[n] = -1; }
-            }
-            if (n >= SERIAL_CAP) atomicOr(d.status, BW_FLAG_EVENT_OVERFLOW);
-            for (int i = 1; i < n; i++) {
-                int s = s_chain[i], q = s_src[i], p = f.pid[s], j = i - 1;
-                while (j >= 0 && f.pid[s_chain[j]] > p) {
-                    s_chain[j + 1] = s_chain[j];
-                    s_src[j + 1] = s_src[j];
-                    j--;
-                }
-                s_chain[j + 1] = s;
-                s_src[j + 1] = q;
-            }
-            s_nser = n;
-        }
-        __syncthreads();
-        const int nser = s_nser;
-        for (int i = 0; i < nser; i++) {
-            const int s = s_chain[i], q = s_src[i];
-            int cx, cy, cz;
-            unpack_cell(f.cell[s], cx, cy, cz);
-            // colloids whose stencil holds the particle's binned cell, ascending
-            const int from = q >= 0 ? d.cont_from[q] : R.first_colloid;
-            if (threadIdx.x == 0) s_cand_n = 0;
-            __syncthreads();
-            for (int base = from; base < gend; base += blockDim.x) {
-                int gg = base + threadIdx.x;
-                bool p = gg < gend && !(ph.surrogate && d.cmode[gg]) &&
-                         in_stencil(cx, cy, cz, d.ccell[3 * gg], d.ccell[3 * gg + 1], d.ccell[3 * gg + 2], L);
-                int tot;
-                int idx = block_compact(p, s_wt, tot);
-                if (p && s_cand_n + idx < TCL_CAP) s_cand[s_cand_n + idx] = gg;
-                __syncthreads();
-                if (threadIdx.x == 0) {
-                    // more candidate colloids than the list holds: the replay
-                    // would miss collisions, so the capacity error is raised
-                    if (s_cand_n + tot > TCL_CAP) atomicOr(d.status, BW_FLAG_LIST_OVERFLOW);
-                    s_cand_n = min(s_cand_n + tot, TCL_CAP);
-                }
-                __syncthreads();
-            }
-            if (threadIdx.x == 0) {
-                const int p = f.pid[s];
-                double bx = f.ox[s], by = f.oy[s], bz = f.oz[s];
-                double vx = f.vx[s], vy = f.vy[s], vz = f.vz[s];
-                double dump[3] = {vx, vy, vz};
-                if (q >= 0)
-                    for (int kk = 0; kk < 3; kk++) dump[kk] = d.cont_dump[3 * q + kk];
-                for (int m = 0; m < s_cand_n; m++) {
-                    const int gg = s_cand[m];
-                    const double *pc = d.cpos + 3 * gg;
-                    double ax = (double)cx + bx, ay = (double)cy + by, az = (double)cz + bz;
-                    double rx = img1(pc[0] - ax, Ld), ry = img1(pc[1] - ay, Ld), rz = img1(pc[2] - az, Ld);
-                    if ((rx * rx + ry * ry) + rz * rz > ph.lim_coll) continue;
-                    ReflDraw dr;
-                    if (!draw_reflection(d, ph, R, step, substep, gg, p, dr)) {
-                        atomicOr(d.status, BW_FLAG_DRAW_MISSING);
-                        continue;
-                    }
-                    double rs[3], c6[6];
-                    reflect_event(ph, L, cx, cy, cz, bx, by, bz, vx, vy, vz, pc, d.cvel + 3 * gg, d.comega + 3 * gg,
-                                  dr, rs, fp32);
-                    transfer(dump, vx, vy, vz, rs, c6);
-                    for (int kk = 0; kk < 3; kk++) {
-                        d.cdv[3 * gg + kk] += c6[kk];
-                        d.cdw[3 * gg + kk] += c6[3 + kk];
-                    }
-                    s_serial_events++;
-                }
-                f.ox[s] = (Real)bx; f.oy[s] = (Real)by; f.oz[s] = (Real)bz;
-                f.vx[s] = (Real)vx; f.vy[s] = (Real)vy; f.vz[s] = (Real)vz;
-            }
-            __syncthreads();
-        }
-    }
-    if (ph.draws == BW_DRAWS_INJECTED) {
-        // every GPU event found its (colloid, particle) tuple; equal totals
-        // then mean equal sets
-        int my_inj = 0;
-        for (int i = threadIdx.x; i < R.nc; i += blockDim.x) {
-            int base = substep * ph.n_colloid_total + R.first_colloid + i;
-            my_inj += d.inj_off[base + 1] - d.inj_off[base];
-        }
-        atomicAdd(&s_inj_tot, my_inj);
-        __syncthreads();
-        if (threadIdx.x == 0 && s_inj_tot != d.ev_total[r] + s_serial_events)
-            atomicOr(d.status, BW_FLAG_DRAW_MISMATCH);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        d.chain_cnt[r] = 0;
-        d.cont_cnt[r] = 0;
-        d.ovf_cnt[r] = 0;
-        d.ev_total[r] = 0;
-    }
+    __shared__ SerialLds s;
+    serial_replay<Real>(ph, d, f, substep, blockIdx.x, true, s);
 }
-
-// ----------------------------------------------------- colloid update (fused)
-// One wave per colloid: collision impulse, orientation, WCA force (the pair
-// addends k_collide stored with this substep's pair list, summed in list
-// order by lane 0), velocity, [run() kick], old force, position into the
-// other buffer.  Follows k_collide of the same substep.
 __global__ __launch_bounds__(256) void k_colloid_update(Phys ph, Dev d, unsigned flags, const int2 *wgt) {
-    __shared__ double s_f[4][MD_CAP][3];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ UpdateLds s[4];
+    const int w = threadIdx.x >> 6;
     const int2 wt = ph.n_rep == 1 ? make_int2(0, blockIdx.x * 4) : wgt[blockIdx.x];
-    const int r = wt.x;
-    const int g = wt.y + w;
-    // Loads that do not need the replica record go first, at an in-range
-    // index (a workgroup's last colloids may lie past its replica); the first
-    // 64 force addends are requested before their count arrives.
-    const int gs = min(g, ph.n_colloid_total - 1);
-    ColIn in;  // lane 0: the colloid's own state, in flight with the force terms
-    if (lane == 0) colloid_load(ph, d, gs, flags, in);
-    int nmd_s = 0;
-    double tl[3] = {0, 0, 0};
-    if (flags & PH_FORCE) {
-        nmd_s = d.md_cnt[gs];
-        for (int k = 0; k < 3; k++) tl[k] = d.md_f[3 * (gs * MD_CAP + lane) + k];
-    }
-    // lanes 0-5: sin (lanes 0-2) or cos (lanes 3-5) of the activity rotation
-    // angle about axis lane % 3, from the angular velocity after the impulse,
-    // formed as colloid_update forms them; lane 0 gathers them below
-    double tv = 0.0;
-    if ((flags & PH_ACTIVITY) && lane < 6) {
-        const int k = lane % 3;
-        double wk = d.comega[3 * gs + k];
-        if (flags & PH_APPLY) {
-            const double iw = (ph.surrogate && d.cmode[gs]) ? d.csur[6 * gs + 3 + k] : d.cdw[3 * gs + k];
-            wk = wk + iw * ph.mass_fl / ph.I_colloid;
-        }
-        const double b = wk * ph.dt;
-        tv = lane < 3 ? sin(b) : cos(b);
-    }
-    const Rep R = d.rep[r];
-    const bool valid = g < R.first_colloid + R.nc;
-    int nmd = 0;
-    if (valid && (flags & PH_FORCE)) {
-        nmd = nmd_s;
-        for (int m = lane; m < nmd; m += 64)
-            for (int k = 0; k < 3; k++) s_f[w][m][k] = m < 64 ? tl[k] : d.md_f[3 * (g * MD_CAP + m) + k];
-    }
-    double trig[6];
-    for (int k = 0; k < 6; k++) trig[k] = __shfl(tv, k);
-    __syncthreads();
-    if (valid && lane == 0) {
-        double fn[3] = {0, 0, 0};
-        if (flags & PH_FORCE) {
-            double f0 = 0, f1 = 0, f2 = 0;
-#pragma unroll 4
-            for (int m = 0; m < nmd; m++) {  // cpp/update.cpp:28 in list order
-                f0 = f0 + s_f[w][m][0];
-                f1 = f1 + s_f[w][m][1];
-                f2 = f2 + s_f[w][m][2];
-            }
-            fn[0] = f0; fn[1] = f1; fn[2] = f2;
-        }
-        colloid_update(ph, d, R.L, r, g, flags, fn, in, (flags & PH_ACTIVITY) ? trig : nullptr);
-    }
+    colloid_update_wave(ph, d, flags, wt.x, wt.y + w, s[w]);
 }
 
 // ------------------------------------------------------- run() (standalone)
@@ -2409,7 +2132,7 @@ __global__ __launch_bounds__(256) void k_sur_shell_kick(Phys ph, Dev d, Fluid<Re
     const int L = d.rep[d.tile_rep[T]].L;
     for (int q = threadIdx.x; q < ns; q += blockDim.x) {
         const int g = d.tsl_list[T * TCL_CAP + q];
-        const ShellPay pay = shell_pay(ph, d, g);
+        const ShellPay pay = shell_pay(ph, d, g, d.cra + 3 * g);
         for (int k = 0; k < 3; k++) {
             s_k[q][k] = d.cpos[3 * g + k];
             s_k[q][3 + k] = pay.u[k];
@@ -2579,6 +2302,11 @@ hipError_t prepare_kernels(Phys &ph, bool fp64) {
         e = fp64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_stream_near<double, false>, 256, 0)
                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_stream_near<float, false>, 256, 0);
     if (e != hipSuccess) return e;
+    int cls_cu = 0;
+    e = fp64 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&cls_cu, k_classify<double>, 256, 0)
+             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&cls_cu, k_classify<float>, 256, 0);
+    if (e != hipSuccess) return e;
+    ph.classify_blocks = std::max(1, std::min(NEAR_BLOCKS, cus * std::max(cls_cu, 1)));
     ph.near_blocks = std::max(1, std::min(NEAR_BLOCKS, cus * std::max(per_cu, 1)));
     return hipSuccess;
 }
@@ -2616,6 +2344,10 @@ template <class Real>
 void launch_stream_near(const Phys &ph, const Dev &d, const Fluid<Real> &f, bool kick, hipStream_t st) {
     if (kick) LAUNCH((k_stream_near<Real, true>), ph.near_blocks, 256, 0, st, ph, d, f);
     else LAUNCH((k_stream_near<Real, false>), ph.near_blocks, 256, 0, st, ph, d, f);
+}
+template <class Real>
+void launch_classify(const Phys &ph, const Dev &d, const Fluid<Real> &f, hipStream_t st) {
+    LAUNCH(k_classify<Real>, ph.classify_blocks, 256, 0, st, ph, d, f);
 }
 template <class Real>
 void launch_collide(const Phys &ph, const Dev &d, const Fluid<Real> &f, int substep, const int2 *wgt, int nwg,
@@ -2659,8 +2391,8 @@ void launch_colloid(const Phys &ph, const Dev &d, unsigned flags, hipStream_t st
 void launch_colloid_update(const Phys &ph, const Dev &d, unsigned flags, const int2 *wgt, int nwg, hipStream_t st) {
     LAUNCH(k_colloid_update, nwg, 256, 0, st, ph, d, flags, wgt);
 }
-void launch_md_candidates(const Phys &ph, const Dev &d, const int2 *wgt, int nwg, hipStream_t st) {
-    LAUNCH(k_md_candidates, nwg, 256, 0, st, ph, d, wgt);
+void launch_md_candidates(const Phys &ph, const Dev &d, const int2 *wgt, int nwg, bool link, hipStream_t st) {
+    LAUNCH(k_md_candidates, nwg, 256, 0, st, ph, d, wgt, (int)link);
 }
 void launch_tile_colloids(const Phys &ph, const Dev &d, hipStream_t st, bool cleared) {
     if (!cleared) LAUNCH(k_tile_lists_clear, (ph.n_tiles + 255) / 256, 256, 0, st, ph, d);
@@ -2735,6 +2467,7 @@ void launch_copy(const void *a, void *b, long long nbytes, hipStream_t st) {
     template void launch_collide<Real>(const Phys &, const Dev &, const Fluid<Real> &, int, const int2 *, int,    \
                                        hipStream_t);                                                               \
     template void launch_stream_near<Real>(const Phys &, const Dev &, const Fluid<Real> &, bool, hipStream_t);    \
+    template void launch_classify<Real>(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);              \
     template void launch_run_count<Real>(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);            \
     template void launch_maps<Real>(const Phys &, const Dev &, const Fluid<Real> &, long long, int *,             \
                                     const int *, hipStream_t);                                                     \
