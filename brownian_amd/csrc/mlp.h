@@ -13,11 +13,14 @@ constexpr int MLP_L = 4;
 // activations of one forward/backward pass over up to `cap` rows
 struct MlpBuf {
     int cap = 0;
-    unsigned short *Xb = nullptr, *Hb[3] = {}, *dYb = nullptr, *dZb = nullptr;
-    float *Z[3] = {}, *H[3] = {}, *Y = nullptr, *dY = nullptr, *dH = nullptr, *dZ = nullptr, *loss = nullptr;
-    float *part = nullptr;  // partial sums of the backward reductions (split-K products, column sums)
+    unsigned short *Xb = nullptr, *Hb[3] = {};
+    float *Y = nullptr;
+    // training only: pre-activations, output gradients, two layers' dZ in turn,
+    // losses, partial sums of the parameter gradients
+    unsigned short *dYb = nullptr, *dZb[2] = {};
+    float *Z[3] = {}, *dY = nullptr, *dZ[2] = {}, *loss = nullptr, *part = nullptr;
 };
-int mlp_buf_alloc(MlpBuf &b, int rows);  // hipMalloc; 0 on success
+int mlp_buf_alloc(MlpBuf &b, int rows, bool train = false);  // hipMalloc; 0 on success
 void mlp_buf_free(MlpBuf &b);
 
 // features x (n x 144 raw units, device) -> y_out (n x 12, device): impulse
