@@ -33,11 +33,12 @@ void launch_collide(const Phys &, const Dev &, const Fluid<Real> &, int, const i
 template <class Real> void launch_run_count(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);
 template <class Real>
 void launch_maps(const Phys &, const Dev &, const Fluid<Real> &, long long, int *, const int *, hipStream_t);
-template <class Real> void launch_audit(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);
+template <class Real> void launch_audit(const Phys &, const Dev &, const Fluid<Real> &, int, int, hipStream_t);
 template <class Real>
-void launch_gather(const Phys &, const Dev &, const Fluid<Real> &, double *, double *, int *, hipStream_t);
+void launch_gather(const Phys &, const Dev &, const Fluid<Real> &, double *, double *, int *, int, int, hipStream_t);
 void launch_step_begin(const Phys &, const Dev &, hipStream_t, bool clear_lists = false);
 void launch_colloid(const Phys &, const Dev &, unsigned, hipStream_t);
+void launch_potential(const Phys &, const Dev &, int, hipStream_t);
 void launch_colloid_update(const Phys &, const Dev &, unsigned, const int2 *, int, hipStream_t);
 void launch_md_candidates(const Phys &, const Dev &, const int2 *, int, bool link, hipStream_t);
 template <class Real> void launch_classify(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);
@@ -909,7 +910,7 @@ int download_fluid_impl(bw_ctx *c, int r, double *pos, double *vel, int *cell) {
             return rc;
     }
     launch_gather<Real>(c->ph, dev_for(c, c->cur), fluid_of<Real>(c, c->cur), c->stage_pos, c->stage_vel,
-                        c->stage_cell, c->st);
+                        c->stage_cell, R.first_tile, R.n_tiles, c->st);
     HIPCHK(c, hipStreamSynchronize(c->st));
     size_t off = (size_t)R.first_fluid;
     if (pos) HIPCHK(c, hipMemcpy(pos, c->stage_pos + 3 * off, sizeof(double) * 3 * R.nf, hipMemcpyDeviceToHost));
@@ -1263,8 +1264,12 @@ BW_API int updown_velocity(bw_ctx *c) {
                         (rc = dalloc(c, &c->ud_upcnt, NC))))
         return rc;
     Dev d = dev_for(c, c->cur);
-    if (c->fp64) launch_gather<double>(c->ph, d, c->fl[c->cur].f64, c->stage_pos, c->stage_vel, c->stage_cell, c->st);
-    else launch_gather<float>(c->ph, d, c->fl[c->cur].f32, c->stage_pos, c->stage_vel, c->stage_cell, c->st);
+    if (c->fp64)
+        launch_gather<double>(c->ph, d, c->fl[c->cur].f64, c->stage_pos, c->stage_vel, c->stage_cell, 0,
+                              c->ph.n_tiles, c->st);
+    else
+        launch_gather<float>(c->ph, d, c->fl[c->cur].f32, c->stage_pos, c->stage_vel, c->stage_cell, 0,
+                             c->ph.n_tiles, c->st);
     launch_updown(c->ph, d, c->n_rep, c->stage_pos, c->stage_vel, c->ud_sums, c->ud_cnt, c->ud_upcnt, c->ud_vel,
                   c->ud_up, c->st);
     return BW_OK;
@@ -1537,20 +1542,31 @@ BW_API int bw_get_run_counts(bw_ctx *c, int r, int *cnt) {
 }
 
 // ------------------------------------------------------------------ audit
+namespace {
+// FP64 sums over replica R's fluid: s[0..2] velocity, s[3] its square, s[4] its
+// absolute components (unit mass)
+int fluid_sums(bw_ctx *c, const ReplicaHost &R, double *s) {
+    const Dev d = dev_for(c, c->cur);
+    if (c->fp64) launch_audit<double>(c->ph, d, c->fl[c->cur].f64, R.first_tile, R.n_tiles, c->st);
+    else launch_audit<float>(c->ph, d, c->fl[c->cur].f32, R.first_tile, R.n_tiles, c->st);
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    std::vector<double> part((size_t)R.n_tiles * 8);
+    HIPCHK(c, hipMemcpy(part.data(), c->dv.audit_partial + (size_t)R.first_tile * 8, sizeof(double) * part.size(),
+                        hipMemcpyDeviceToHost));
+    for (int k = 0; k < 5; k++) s[k] = 0;
+    for (int t = 0; t < R.n_tiles; t++)
+        for (int k = 0; k < 5; k++) s[k] += part[(size_t)t * 8 + k];
+    return BW_OK;
+}
+}  // namespace
+
 BW_API int bw_audit(bw_ctx *c, int r, double *out) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !out) return BW_ERR_ARG;
-    Dev d = dev_for(c, c->cur);
-    if (c->fp64) launch_audit<double>(c->ph, d, c->fl[c->cur].f64, c->st);
-    else launch_audit<float>(c->ph, d, c->fl[c->cur].f32, c->st);
-    launch_colloid(c->ph, d, PH_POTENTIAL, c->st);
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    std::vector<double> part((size_t)R->n_tiles * 8);
-    HIPCHK(c, hipMemcpy(part.data(), c->dv.audit_partial + (size_t)R->first_tile * 8, sizeof(double) * part.size(),
-                        hipMemcpyDeviceToHost));
-    double s[5] = {0, 0, 0, 0, 0};
-    for (int t = 0; t < R->n_tiles; t++)
-        for (int k = 0; k < 5; k++) s[k] += part[(size_t)t * 8 + k];
+    if (R->nc) launch_potential(c->ph, dev_for(c, c->cur), r, c->st);
+    double s[5];
+    const int rc = fluid_sums(c, *R, s);  // synchronises
+    if (rc) return rc;
     std::vector<double> v(3 * R->nc), w(3 * R->nc);
     double pot = 0;
     if (R->nc) {
@@ -1629,13 +1645,14 @@ BW_API int bw_observables_reset(bw_ctx *c) {
 BW_API int bw_observables(bw_ctx *c, int r, double *out) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !out) return BW_ERR_ARG;
-    double a[11];
-    int rc = bw_audit(c, r, a);  // synchronises; FP64 fluid sums
+    double s[5];
+    const int rc = fluid_sums(c, *R, s);  // synchronises
     if (rc) return rc;
     const double m = R->p.mass_fl, N = (double)R->nf;
-    const double p2 = a[7] * a[7] + a[8] * a[8] + a[9] * a[9];  // |m sum v|^2
+    const double ke = 0.5 * s[3] * m, px = s[0] * m, py = s[1] * m, pz = s[2] * m;
+    const double p2 = px * px + py * py + pz * pz;  // |m sum v|^2
     out[0] = (double)(c->steps_done - R->obs_step0);
-    out[3] = R->nf > 1 ? (2.0 * a[3] - p2 / (N * m)) / (3.0 * (N - 1.0)) : 0.0;
+    out[3] = R->nf > 1 ? (2.0 * ke - p2 / (N * m)) / (3.0 * (N - 1.0)) : 0.0;
     out[1] = out[2] = out[4] = out[5] = 0.0;
     if (R->nc) {
         size_t n3 = 3 * (size_t)R->nc, o = 3 * (size_t)R->first_colloid;

@@ -58,7 +58,6 @@ enum : unsigned {
     PH_OLDF = 1u << 5,      // cpp/active_brownian.cpp:28
     PH_POS = 1u << 6,       // cpp/update.cpp:48-54
     PH_MDLIST = 1u << 7,    // filter candidates into the pair list (cpp/neighbour_list.cpp:27-39)
-    PH_POTENTIAL = 1u << 8, // potential in the reference's summation order
     PH_RESET_EVENTS = 1u << 9,
     PH_MARGIN = 1u << 10,   // check the colloid displacement bound of blocked streaming
 };

@@ -1041,27 +1041,6 @@ __device__ inline void colloid_phases(const Phys &ph, const Dev &d, const Rep &R
     if (flags & PH_MDLIST)
         for (int i = threadIdx.x; i < nc; i += blockDim.x) colloid_mdlist_serial(ph, d, R, r, g0 + i);
     __syncthreads();
-    if (flags & PH_POTENTIAL) {
-        // cpp/update.cpp:24, one running sum over (i ascending, j > i ascending)
-        if (threadIdx.x == 0) {
-            double pot = 0;
-            for (int i = 0; i < nc; i++) {
-                int g = g0 + i;
-                for (int m = 0; m < d.md_cnt[g]; m++) {
-                    int j = d.md_list[g * MD_CAP + m];
-                    if (j <= g) continue;
-                    const double *pi = d.cpos + 3 * g, *pj = d.cpos + 3 * j;
-                    double tx = img1(pi[0] - pj[0], L), ty = img1(pi[1] - pj[1], L), tz = img1(pi[2] - pj[2], L);
-                    double rr = sqrt((tx * tx + ty * ty) + tz * tz);
-                    if (rr < ph.r_cutoff)
-                        pot += 4 * ph.eps * (pow(ph.sig_colloid / rr, 12) - pow(ph.sig_colloid / rr, 6)) - ph.ufc +
-                               ph.fc * rr;
-                }
-            }
-            d.cpot[r] = pot;
-        }
-    }
-    __syncthreads();
 }
 
 }  // namespace bw

@@ -1985,10 +1985,13 @@ __global__ void k_updown_finish(Dev d, const double *sums, int *cnt, int *up_cnt
 }
 
 // ------------------------------------------------------------------- audit
+// FP64 sums over each tile of one replica (tiles first, first + 1, ...; the
+// host adds the tiles in order).  A context of many replicas is audited one
+// replica at a time, so the grid is that replica's tiles only.
 template <class Real>
-__global__ void k_audit(Phys ph, Dev d, Fluid<Real> f) {
+__global__ void k_audit(Phys ph, Dev d, Fluid<Real> f, int first) {
     __shared__ double s[256][5];
-    const int T = blockIdx.x;
+    const int T = first + blockIdx.x;
     const int n = min(d.count[T], ph.cap);
     double a[5] = {0, 0, 0, 0, 0};
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
@@ -2008,10 +2011,49 @@ __global__ void k_audit(Phys ph, Dev d, Fluid<Real> f) {
     if (threadIdx.x < 5) d.audit_partial[T * 8 + threadIdx.x] = s[0][threadIdx.x];
 }
 
+// The WCA potential of one replica in the reference's order: one running sum
+// over (i ascending, j > i ascending), cpp/update.cpp:24.  The terms of 32
+// colloids at a time are formed by eight threads each and added by one thread,
+// in that order (a pair that does not count adds 0, which changes no sum): two
+// pow() per pair in one thread were 7.0 ms at 2400 colloids.
+__global__ __launch_bounds__(256) void k_potential(Phys ph, Dev d, int r) {
+    constexpr int NB = 32, TPC = 256 / NB;
+    __shared__ double s_term[NB][MD_CAP];
+    __shared__ int s_cnt[NB];
+    const Rep R = d.rep[r];
+    const double L = (double)R.L;
+    const int q = threadIdx.x / TPC, lane = threadIdx.x % TPC;
+    double pot = 0;
+    for (int b = 0; b < R.nc; b += NB) {
+        const int g = R.first_colloid + b + q;
+        const int cnt = b + q < R.nc ? d.md_cnt[g] : 0;
+        if (lane == 0) s_cnt[q] = cnt;
+        for (int m = lane; m < cnt; m += TPC) {
+            const int j = d.md_list[g * MD_CAP + m];
+            double term = 0;
+            if (j > g) {
+                const double *pi = d.cpos + 3 * g, *pj = d.cpos + 3 * j;
+                const double tx = img1(pi[0] - pj[0], L), ty = img1(pi[1] - pj[1], L), tz = img1(pi[2] - pj[2], L);
+                const double rr = sqrt((tx * tx + ty * ty) + tz * tz);
+                if (rr < ph.r_cutoff)
+                    term = 4 * ph.eps * (pow(ph.sig_colloid / rr, 12) - pow(ph.sig_colloid / rr, 6)) - ph.ufc +
+                           ph.fc * rr;
+            }
+            s_term[q][m] = term;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0)
+            for (int i = 0; i < min(NB, R.nc - b); i++)
+                for (int m = 0; m < s_cnt[i]; m++) pot += s_term[i][m];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) d.cpot[r] = pot;
+}
+
 // ------------------------------------------------------- gather (download)
 template <class Real>
-__global__ void k_gather(Phys ph, Dev d, Fluid<Real> f, double *pos, double *vel, int *cell) {
-    const int T = blockIdx.x;
+__global__ void k_gather(Phys ph, Dev d, Fluid<Real> f, double *pos, double *vel, int *cell, int first) {
+    const int T = first + blockIdx.x;
     Rep R;
     TileGeo tg = tile_geo(d, T, R);
     const int L = tg.L;
@@ -2374,13 +2416,16 @@ void launch_maps(const Phys &ph, const Dev &d, const Fluid<Real> &f, long long n
     if (ph.n_colloid_total > 0) LAUNCH(k_neigh_fl, ph.n_colloid_total, 256, 0, st, ph, d, colloid_rep);
 }
 template <class Real>
-void launch_audit(const Phys &ph, const Dev &d, const Fluid<Real> &f, hipStream_t st) {
-    LAUNCH(k_audit<Real>, ph.n_tiles, 256, 0, st, ph, d, f);
+void launch_audit(const Phys &ph, const Dev &d, const Fluid<Real> &f, int first, int n, hipStream_t st) {
+    LAUNCH(k_audit<Real>, n, 256, 0, st, ph, d, f, first);
+}
+void launch_potential(const Phys &ph, const Dev &d, int r, hipStream_t st) {
+    LAUNCH(k_potential, 1, 256, 0, st, ph, d, r);
 }
 template <class Real>
-void launch_gather(const Phys &ph, const Dev &d, const Fluid<Real> &f, double *pos, double *vel, int *cell,
-                   hipStream_t st) {
-    LAUNCH(k_gather<Real>, ph.n_tiles, 256, 0, st, ph, d, f, pos, vel, cell);
+void launch_gather(const Phys &ph, const Dev &d, const Fluid<Real> &f, double *pos, double *vel, int *cell, int first,
+                   int n, hipStream_t st) {
+    LAUNCH(k_gather<Real>, n, 256, 0, st, ph, d, f, pos, vel, cell, first);
 }
 void launch_step_begin(const Phys &ph, const Dev &d, hipStream_t st, bool clear_lists) {
     LAUNCH(k_step_begin, clear_lists ? std::max(1, (ph.n_tiles + 255) / 256) : 1, 256, 0, st, ph, d, (int)clear_lists);
@@ -2471,9 +2516,9 @@ void launch_copy(const void *a, void *b, long long nbytes, hipStream_t st) {
     template void launch_run_count<Real>(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);            \
     template void launch_maps<Real>(const Phys &, const Dev &, const Fluid<Real> &, long long, int *,             \
                                     const int *, hipStream_t);                                                     \
-    template void launch_audit<Real>(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);                \
+    template void launch_audit<Real>(const Phys &, const Dev &, const Fluid<Real> &, int, int, hipStream_t);      \
     template void launch_gather<Real>(const Phys &, const Dev &, const Fluid<Real> &, double *, double *, int *,  \
-                                      hipStream_t);
+                                      int, int, hipStream_t);
 INST(float)
 INST(double)
 
