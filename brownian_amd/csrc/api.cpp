@@ -13,6 +13,7 @@
 #include "bw_common.h"
 #include "host_init.h"
 #include "mlp.h"
+#include "staging.h"
 
 namespace bw {
 // kernel launchers (kernels.hip)
@@ -122,6 +123,7 @@ struct bw_ctx {
     size_t srd_lds = 0;
     bool maps_alloc = false;
     double *stage_pos = nullptr, *stage_vel = nullptr;
+    Staging staging;
     // updown_velocity results: per-colloid sums, counts and velocities
     double *ud_sums = nullptr, *ud_vel = nullptr, *ud_up = nullptr;
     int *ud_cnt = nullptr, *ud_upcnt = nullptr;
@@ -911,11 +913,11 @@ int download_fluid_impl(bw_ctx *c, int r, double *pos, double *vel, int *cell) {
     }
     launch_gather<Real>(c->ph, dev_for(c, c->cur), fluid_of<Real>(c, c->cur), c->stage_pos, c->stage_vel,
                         c->stage_cell, R.first_tile, R.n_tiles, c->st);
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    size_t off = (size_t)R.first_fluid;
-    if (pos) HIPCHK(c, hipMemcpy(pos, c->stage_pos + 3 * off, sizeof(double) * 3 * R.nf, hipMemcpyDeviceToHost));
-    if (vel) HIPCHK(c, hipMemcpy(vel, c->stage_vel + 3 * off, sizeof(double) * 3 * R.nf, hipMemcpyDeviceToHost));
-    if (cell) HIPCHK(c, hipMemcpy(cell, c->stage_cell + off, sizeof(int) * R.nf, hipMemcpyDeviceToHost));
+    const size_t off = (size_t)R.first_fluid, n = (size_t)R.nf;
+    const StageSeg seg[] = {{pos, c->stage_pos + 3 * off, sizeof(double) * 3 * n},
+                            {vel, c->stage_vel + 3 * off, sizeof(double) * 3 * n},
+                            {cell, c->stage_cell + off, sizeof(int) * n}};
+    HIPCHK(c, c->staging.download(seg, 3, c->st));
     return BW_OK;
 }
 
@@ -1400,25 +1402,18 @@ BW_API int bw_download_colloid(bw_ctx *c, int r, double *pos, double *vel, doubl
                                double *ra) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    size_t o = 3 * (size_t)R->first_colloid, n = sizeof(double) * 3 * R->nc;
-    if (!R->nc) return BW_OK;
-    if (pos) HIPCHK(c, hipMemcpy(pos, c->cposb[c->cb] + o, n, hipMemcpyDeviceToHost));
-    if (vel) HIPCHK(c, hipMemcpy(vel, c->dv.cvel + o, n, hipMemcpyDeviceToHost));
-    if (omega) HIPCHK(c, hipMemcpy(omega, c->dv.comega + o, n, hipMemcpyDeviceToHost));
-    if (f) HIPCHK(c, hipMemcpy(f, c->dv.cf + o, n, hipMemcpyDeviceToHost));
-    if (old_f) HIPCHK(c, hipMemcpy(old_f, c->dv.coldf + o, n, hipMemcpyDeviceToHost));
-    if (ra) HIPCHK(c, hipMemcpy(ra, c->dv.cra + o, n, hipMemcpyDeviceToHost));
+    const size_t o = 3 * (size_t)R->first_colloid, n = sizeof(double) * 3 * R->nc;
+    const StageSeg seg[] = {{pos, c->cposb[c->cb] + o, n}, {vel, c->dv.cvel + o, n},   {omega, c->dv.comega + o, n},
+                            {f, c->dv.cf + o, n},          {old_f, c->dv.coldf + o, n}, {ra, c->dv.cra + o, n}};
+    HIPCHK(c, c->staging.download(seg, 6, c->st));
     return BW_OK;
 }
 
 BW_API int bw_download_displacement(bw_ctx *c, int r, double *disp) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !disp) return BW_ERR_ARG;
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    if (R->nc)
-        HIPCHK(c, hipMemcpy(disp, c->dv.cdisp + 3 * (size_t)R->first_colloid, sizeof(double) * 3 * R->nc,
-                            hipMemcpyDeviceToHost));
+    const StageSeg seg = {disp, c->dv.cdisp + 3 * (size_t)R->first_colloid, sizeof(double) * 3 * R->nc};
+    HIPCHK(c, c->staging.download(&seg, 1, c->st));
     return BW_OK;
 }
 
@@ -1544,15 +1539,15 @@ BW_API int bw_get_run_counts(bw_ctx *c, int r, int *cnt) {
 // ------------------------------------------------------------------ audit
 namespace {
 // FP64 sums over replica R's fluid: s[0..2] velocity, s[3] its square, s[4] its
-// absolute components (unit mass)
-int fluid_sums(bw_ctx *c, const ReplicaHost &R, double *s) {
+// absolute components (unit mass); the transfer takes the n_more segments along
+int fluid_sums(bw_ctx *c, const ReplicaHost &R, double *s, const StageSeg *more, int n_more) {
     const Dev d = dev_for(c, c->cur);
     if (c->fp64) launch_audit<double>(c->ph, d, c->fl[c->cur].f64, R.first_tile, R.n_tiles, c->st);
     else launch_audit<float>(c->ph, d, c->fl[c->cur].f32, R.first_tile, R.n_tiles, c->st);
-    HIPCHK(c, hipStreamSynchronize(c->st));
     std::vector<double> part((size_t)R.n_tiles * 8);
-    HIPCHK(c, hipMemcpy(part.data(), c->dv.audit_partial + (size_t)R.first_tile * 8, sizeof(double) * part.size(),
-                        hipMemcpyDeviceToHost));
+    StageSeg seg[PackSegs::MAX] = {{part.data(), c->dv.audit_partial + (size_t)R.first_tile * 8, sizeof(double) * part.size()}};
+    std::copy(more, more + n_more, seg + 1);
+    HIPCHK(c, c->staging.download(seg, 1 + n_more, c->st));
     for (int k = 0; k < 5; k++) s[k] = 0;
     for (int t = 0; t < R.n_tiles; t++)
         for (int k = 0; k < 5; k++) s[k] += part[(size_t)t * 8 + k];
@@ -1564,16 +1559,14 @@ BW_API int bw_audit(bw_ctx *c, int r, double *out) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !out) return BW_ERR_ARG;
     if (R->nc) launch_potential(c->ph, dev_for(c, c->cur), r, c->st);
-    double s[5];
-    const int rc = fluid_sums(c, *R, s);  // synchronises
+    const size_t n3 = 3 * (size_t)R->nc, o = 3 * (size_t)R->first_colloid;
+    std::vector<double> v(n3), w(n3);
+    double pot = 0, s[5];
+    const StageSeg seg[] = {{v.data(), c->dv.cvel + o, sizeof(double) * n3},
+                            {w.data(), c->dv.comega + o, sizeof(double) * n3},
+                            {&pot, c->dv.cpot + r, R->nc ? sizeof(double) : 0}};
+    const int rc = fluid_sums(c, *R, s, seg, 3);
     if (rc) return rc;
-    std::vector<double> v(3 * R->nc), w(3 * R->nc);
-    double pot = 0;
-    if (R->nc) {
-        HIPCHK(c, hipMemcpy(v.data(), c->dv.cvel + 3 * R->first_colloid, sizeof(double) * v.size(), hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(w.data(), c->dv.comega + 3 * R->first_colloid, sizeof(double) * w.size(), hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(&pot, c->dv.cpot + r, sizeof(double), hipMemcpyDeviceToHost));
-    }
     double kec = 0, ang = 0, pc[3] = {0, 0, 0}, absm = 0;
     for (int i = 0; i < R->nc; i++) {
         kec += (v[3 * i] * v[3 * i] + v[3 * i + 1] * v[3 * i + 1]) + v[3 * i + 2] * v[3 * i + 2];
@@ -1645,8 +1638,14 @@ BW_API int bw_observables_reset(bw_ctx *c) {
 BW_API int bw_observables(bw_ctx *c, int r, double *out) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !out) return BW_ERR_ARG;
+    const size_t n3 = 3 * (size_t)R->nc, o = 3 * (size_t)R->first_colloid;
+    std::vector<double> d(n3), ra(n3), v(n3), w(n3);
+    const StageSeg seg[] = {{d.data(), c->dv.cdisp + o, sizeof(double) * n3},
+                            {ra.data(), c->dv.cra + o, sizeof(double) * n3},
+                            {v.data(), c->dv.cvel + o, sizeof(double) * n3},
+                            {w.data(), c->dv.comega + o, sizeof(double) * n3}};
     double s[5];
-    const int rc = fluid_sums(c, *R, s);  // synchronises
+    const int rc = fluid_sums(c, *R, s, seg, 4);
     if (rc) return rc;
     const double m = R->p.mass_fl, N = (double)R->nf;
     const double ke = 0.5 * s[3] * m, px = s[0] * m, py = s[1] * m, pz = s[2] * m;
@@ -1655,12 +1654,6 @@ BW_API int bw_observables(bw_ctx *c, int r, double *out) {
     out[3] = R->nf > 1 ? (2.0 * ke - p2 / (N * m)) / (3.0 * (N - 1.0)) : 0.0;
     out[1] = out[2] = out[4] = out[5] = 0.0;
     if (R->nc) {
-        size_t n3 = 3 * (size_t)R->nc, o = 3 * (size_t)R->first_colloid;
-        std::vector<double> d(n3), ra(n3), v(n3), w(n3);
-        HIPCHK(c, hipMemcpy(d.data(), c->dv.cdisp + o, sizeof(double) * n3, hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(ra.data(), c->dv.cra + o, sizeof(double) * n3, hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(v.data(), c->dv.cvel + o, sizeof(double) * n3, hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(w.data(), c->dv.comega + o, sizeof(double) * n3, hipMemcpyDeviceToHost));
         if (R->ra0.size() != n3) R->ra0 = ra;  // no reset yet: the origin is now
         double msd = 0, oc = 0, tv = 0, tw = 0;
         for (int i = 0; i < R->nc; i++) {

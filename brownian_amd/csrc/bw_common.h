@@ -219,4 +219,12 @@ struct InitBins {
     const double *cpos;        // colloid positions (global)
 };
 
+// device arrays of 32-bit words packed one after another (word off[i] on)
+struct PackSegs {
+    static constexpr int MAX = 8;
+    const int *src[MAX];
+    int off[MAX + 1];
+    int n;
+};
+
 }  // namespace bw

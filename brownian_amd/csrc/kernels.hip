@@ -2050,6 +2050,16 @@ __global__ __launch_bounds__(256) void k_potential(Phys ph, Dev d, int r) {
     if (threadIdx.x == 0) d.cpot[r] = pot;
 }
 
+// Several device arrays one after another into dst, which may be pinned host
+// memory: one launch and one wait in place of a copy per array.  Bound by the
+// launch and the bus (64 KB 15 us, 1 MB 60 us with the wait).
+__global__ __launch_bounds__(256) void k_pack(PackSegs s, int *dst) {
+    for (int q = 0; q < s.n; q++) {
+        const int n = s.off[q + 1] - s.off[q];
+        for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += 256 * gridDim.x) dst[s.off[q] + i] = s.src[q][i];
+    }
+}
+
 // ------------------------------------------------------- gather (download)
 template <class Real>
 __global__ void k_gather(Phys ph, Dev d, Fluid<Real> f, double *pos, double *vel, int *cell, int first) {
@@ -2418,6 +2428,11 @@ void launch_maps(const Phys &ph, const Dev &d, const Fluid<Real> &f, long long n
 template <class Real>
 void launch_audit(const Phys &ph, const Dev &d, const Fluid<Real> &f, int first, int n, hipStream_t st) {
     LAUNCH(k_audit<Real>, n, 256, 0, st, ph, d, f, first);
+}
+void launch_pack(const PackSegs &s, int *dst, hipStream_t st) {
+    int most = 1;
+    for (int q = 0; q < s.n; q++) most = std::max(most, s.off[q + 1] - s.off[q]);
+    LAUNCH(k_pack, std::min(256, (most + 255) / 256), 256, 0, st, s, dst);
 }
 void launch_potential(const Phys &ph, const Dev &d, int r, hipStream_t st) {
     LAUNCH(k_potential, 1, 256, 0, st, ph, d, r);
