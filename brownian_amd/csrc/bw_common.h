@@ -42,6 +42,11 @@ constexpr int N_FEAT = 144;         // surrogate features per colloid
 constexpr int COARSE_MAX = 64;      // coarse cells of one tile
 constexpr int GROUP_SMALL = 1;      // colloids of a group that one wave of k_groups takes
 constexpr int GROUP_MAX = 24;       // colloids of a group that a workgroup of it takes
+// up to here every group gets a workgroup: two on each of 256 CUs run side by
+// side, and four waves take a lone colloid through its step in 100 us in place
+// of 140 (45^3, 77 colloids; a step at 80^3 with 512 colloids 444 against 467
+// us, with 640 already 554 against 485)
+constexpr int GROUP_WIDE = 512;
 constexpr int GROUP_LDS_COLLOIDS = 3072;  // colloids that k_group_lists holds in LDS
 constexpr int OVL_CAP = 65536;      // hot particles beyond a full bucket, all colloids
 constexpr long long MEAN_CHUNK = 65536;  // particles per workgroup of the start-up's mean

@@ -852,7 +852,7 @@ __global__ __launch_bounds__(1024) void k_group_lists(Phys ph, Dev d) {
         if (C > GROUP_MAX) continue;
         const int o = atomicAdd(&s_mem, C);
         d.grp_hot[g] = atomicAdd(&s_hot, hot[g]);
-        if (C > GROUP_SMALL) d.grp_big[atomicAdd(&s_big, 1)] = make_int2(o, C);
+        if (C > GROUP_SMALL || nc <= GROUP_WIDE) d.grp_big[atomicAdd(&s_big, 1)] = make_int2(o, C);
         else d.grp_small[atomicAdd(&s_small, 1)] = make_int2(o, C);
         off[g] = o;
     }
@@ -872,10 +872,13 @@ __global__ __launch_bounds__(1024) void k_group_lists(Phys ph, Dev d) {
     }
 }
 
-// One workgroup per large group, then one wave per small one.  final: the last
-// substep ends with update_velocity_colloid (no kick, no position update).
-template <class Real>
-__global__ __launch_bounds__(256, sizeof(Real) == 4 ? 3 : 2) void k_groups(GroupArgs<Real> a) {
+// One workgroup per large group, then one wave per small one; WIDE: a workgroup
+// for every group (up to GROUP_WIDE colloids).  Two workgroups per CU are all
+// that a WIDE launch has (226 VGPRs, none spilled); the other takes three in
+// FP32 (168, some spilled), which 2400 groups need to run at once.  final: the
+// last substep ends with update_velocity_colloid (no kick, no position update).
+template <class Real, bool WIDE>
+__global__ __launch_bounds__(256, WIDE || sizeof(Real) == 8 ? 2 : 3) void k_groups(GroupArgs<Real> a) {
     const Phys &ph = a.ph;
     const Dev &d = a.d;
     const Fluid<Real> &f = a.f;
@@ -883,9 +886,9 @@ __global__ __launch_bounds__(256, sizeof(Real) == 4 ? 3 : 2) void k_groups(Group
     const int final = a.final;
     __shared__ union {
         GroupLds<Real, 4> big;
-        GroupLds<Real, 1> small[4];
+        GroupLds<Real, 1> small[WIDE ? 1 : 4];
     } s;
-    const int n_big = ld_const(d.grp_cnt), n_small = ld_const(d.grp_cnt + 1);
+    const int n_big = ld_const(d.grp_cnt), n_small = WIDE ? 0 : ld_const(d.grp_cnt + 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // members in ascending order into g[0..C)
     auto members = [&](int2 grp, int *g) {
@@ -904,7 +907,7 @@ __global__ __launch_bounds__(256, sizeof(Real) == 4 ? 3 : 2) void k_groups(Group
         __syncthreads();
         const int r = __builtin_amdgcn_readfirstlane(d.crep[s.big.g[0]]);
         if (!group_step<Real, 4>(ph, d, f, h, final, grp.y, r, s.big)) left(s.big.g, grp.y, r, threadIdx.x, 256);
-    } else {
+    } else if constexpr (!WIDE) {
         const int i = ((int)blockIdx.x - n_big) * 4 + w;
         if (i >= n_small) return;
         const int2 grp = ld_const(d.grp_small + i);
@@ -1107,8 +1110,10 @@ __global__ __launch_bounds__(256) void k_pair_lists(Phys ph, Dev d, const int2 *
 template <class Real>
 void launch_groups(const Phys &ph, const Dev &d, const Fluid<Real> &f, HotPart<Real> *h, bool final, hipStream_t st) {
     hipLaunchKernelGGL(k_group_lists, dim3(1), dim3(1024), 0, st, ph, d);
-    // at most n/2 large groups, or n/4 workgroups of small ones
-    hipLaunchKernelGGL(k_groups<Real>, dim3(ph.n_colloid_total / 2 + 1), dim3(256), 0, st, GroupArgs<Real>{ph, d, f, h, (int)final});
+    // at most n/2 large groups, or n/4 workgroups of small ones (WIDE: n groups)
+    const GroupArgs<Real> a{ph, d, f, h, (int)final};
+    if (ph.n_colloid_total <= GROUP_WIDE) hipLaunchKernelGGL((k_groups<Real, true>), dim3(ph.n_colloid_total), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_groups<Real, false>), dim3(ph.n_colloid_total / 2 + 1), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_groups_redo<Real>, dim3(ph.n_rep), dim3(COLLIDE_THREADS), 0, st, ph, d, f, (int)final);
 }
 template void launch_groups<float>(const Phys &, const Dev &, const Fluid<float> &, HotPart<float> *, bool, hipStream_t);

@@ -91,3 +91,20 @@ def test_groups_equal_per_substep_fp32(case):
     d = a[1][0] - b[1][0]
     d -= a[4] * np.round(d / a[4])
     assert np.abs(d).max() <= 25 * 2.0 ** -24  # n_sub roundings of an offset below 1
+
+
+@pytest.mark.parametrize("replicas", [64, 65])
+def test_many_groups_equal_per_substep(replicas):
+    """512 colloids and more: a workgroup for every group, one wave for lone colloids"""
+    prm = [dict(BASE, L=16, n_colloid=8, n_sub=4, seed=100 + r, precision=B.BW_FP64) for r in range(replicas)]
+    a, b = (B.System(replicas=[dict(p, streaming=s) for p in prm]) for s in (B.BW_STREAM_BLOCKED, B.BW_STREAM_PER_SUBSTEP))
+    for s in (a, b):
+        s.startup()
+        s.step(2)
+        assert s.status() == 0
+    for r in (0, replicas // 2, replicas - 1):
+        for x, y in zip(a.download_fluid(r), b.download_fluid(r)):
+            np.testing.assert_array_equal(x, y)
+        ca, cb = a.download_colloid(r), b.download_colloid(r)
+        for k in ca:
+            np.testing.assert_array_equal(ca[k], cb[k], err_msg=k)
