@@ -292,24 +292,63 @@ __device__ __forceinline__ bool in_unit3(double a, double b, double c) {
 }
 
 
-// one particle streamed through n substeps (cpp/update.cpp:56-60); FLAT: by
-// normalise_flat
-template <bool FLAT, class Real>
+// one particle streamed through n substeps (cpp/update.cpp:56-60)
+template <class Real>
 __device__ __forceinline__ void fly(int n, Real dt, int L, Real vx, Real vy, Real vz, int &ix, int &iy, int &iz,
                                     Real &ox, Real &oy, Real &oz) {
     const Real dx = vx * dt, dy = vy * dt, dz = vz * dt;
-    auto norm = [&](int &i, Real &o) {
-        if constexpr (FLAT) normalise_flat(i, o, L);
-        else normalise(i, o, L);
-    };
     for (int l = 0; l < n; l++) {
         ox = ox + dx;
         oy = oy + dy;
         oz = oz + dz;
-        norm(ix, ox);
-        norm(iy, oy);
-        norm(iz, oz);
+        normalise(ix, ox, L);
+        normalise(iy, oy, L);
+        normalise(iz, oz, L);
     }
+}
+// the same by normalise_flat.  The offsets do not depend on the cells, so where
+// all active lanes move less than a cell per substep the cells crossed are
+// counted and wrapped once at the end
+template <class Real>
+__device__ __forceinline__ void fly_flat(int n, Real dt, int L, Real vx, Real vy, Real vz, int &ix, int &iy, int &iz,
+                                         Real &ox, Real &oy, Real &oz) {
+    const Real dx = vx * dt, dy = vy * dt, dz = vz * dt;
+    if (__ballot(!(fabs(dx) < Real(1) && fabs(dy) < Real(1) && fabs(dz) < Real(1)))) {
+        for (int l = 0; l < n; l++) {
+            ox = ox + dx;
+            oy = oy + dy;
+            oz = oz + dz;
+            normalise_flat(ix, ox, L);
+            normalise_flat(iy, oy, L);
+            normalise_flat(iz, oz, L);
+        }
+        return;
+    }
+    int cx = ix, cy = iy, cz = iz;
+    auto move = [](int &c, Real &o, Real d) {  // normalise_flat without the wrap
+        o = o + d;
+        const Real f = floor(o);
+        const Real q = f != Real(0) ? o - f : o;
+        const bool up = q >= Real(1);
+        o = up ? Real(0) : q;
+        c += (int)f + (up ? 1 : 0);
+    };
+    for (int l = 0; l < n; l++) {
+        move(cx, ox, dx);
+        move(cy, oy, dy);
+        move(cz, oz, dz);
+    }
+    auto wrap = [&](int &i, int c) {
+        c = wrap_once(c, L);
+        if ((unsigned)c >= (unsigned)L) {
+            c %= L;
+            if (c < 0) c += L;
+        }
+        i = c;
+    };
+    wrap(ix, cx);
+    wrap(iy, cy);
+    wrap(iz, cz);
 }
 
 // ------------------------------------------------------------ reflection

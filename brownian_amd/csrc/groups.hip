@@ -197,8 +197,21 @@ __device__ __noinline__ int replay(const GroupArgs<Real> *a, int r, int l, int p
     return n | flags;
 }
 
-// Values of the other axes of a lane's quad (lanes 4i .. 4i+3; axes on the first three)
-__device__ __forceinline__ double quad(double x, int l0, int k) { return __shfl(x, l0 + k); }
+// Values of the other lanes of a lane's quad (lanes 4i .. 4i+3, all active; axes
+// on the first three): lane K's, and those of the next and the previous axis
+// (cyclically; lane 3 as lane 2).  Lane permutes of the ALU: a shuffle by way of
+// the LDS unit is a wait of some 100 cycles in the chain.
+template <int CTRL>
+__device__ __forceinline__ double quad_perm(double x) {
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int K>
+__device__ __forceinline__ double quad(double x) { return quad_perm<0x55 * K>(x); }
+__device__ __forceinline__ double quad_next(double x) { return quad_perm<1 | 2 << 2>(x); }
+__device__ __forceinline__ double quad_prev(double x) { return quad_perm<2 | 1 << 4 | 1 << 6>(x); }
 
 // The stochastic reflection of a particle by a colloid, an axis per lane of a
 // quad (k = 0..2; lane 3 only draws): reflect_event's and draw_reflection's
@@ -222,8 +235,8 @@ __device__ __forceinline__ bool reflect_quad(const Phys &ph, const Rep &R, const
         const uint32_t c0 = KIND_REFL | ((uint32_t)substep << 8), jl = (uint32_t)(g - R.first_colloid);
         uint4 a = philox(make_uint4(c0 | ((uint32_t)k << 16), (uint32_t)step, (uint32_t)pid, jl), rep_key(R));
         double ua = u01(a.x, a.y), ub = u01(a.z, a.w);
-        u_e = __shfl(ua, l0);
-        const double tx = __shfl(ub, l0), ty = __shfl(ua, l0 + 1), tz = __shfl(ub, l0 + 1);
+        u_e = quad<0>(ua);
+        const double tx = quad<0>(ub), ty = quad<1>(ua), tz = quad<1>(ub);
         t_k = k == 0 ? tx : k == 1 ? ty : tz;
         // the polar pair: the first accepted try, four tries per round (the
         // first round's lanes 0 and 1 hold the other draws)
@@ -255,18 +268,17 @@ __device__ __forceinline__ bool reflect_quad(const Phys &ph, const Rep &R, const
     const double z = x1 * x1 + x2 * x2;
     const double lg = log(k == 1 ? z : re);
     const double sq = sqrt((k == 1 ? -2.0 * lg : -lg) / (k == 1 ? z : m_beta));
-    const double val = __shfl(sq, l0), zt = __shfl(sq, l0 + 1);
-    double r0 = quad(rs, l0, 0), r1 = quad(rs, l0, 1), r2 = quad(rs, l0, 2);
+    const double val = quad<0>(sq), zt = quad<1>(sq);
+    double r0 = quad<0>(rs), r1 = quad<1>(rs), r2 = quad<2>(rs);
     const double nrm = sqrt((r0 * r0 + r1 * r1) + r2 * r2);
     const double un = rs / nrm * val;
     const double tk = img1(t_k * Ld - a_k, Ld);
-    const int n1 = k >= 2 ? 0 : k + 1, n2 = k == 0 ? 2 : k == 3 ? 1 : k - 1;  // the next axes, cyclically
-    double ut = quad(un, l0, n1) * quad(tk, l0, n2) - quad(un, l0, n2) * quad(tk, l0, n1);
-    const double q0 = quad(ut, l0, 0), q1 = quad(ut, l0, 1), q2 = quad(ut, l0, 2);
+    double ut = quad_next(un) * quad_prev(tk) - quad_prev(un) * quad_next(tk);
+    const double q0 = quad<0>(ut), q1 = quad<1>(ut), q2 = quad<2>(ut);
     ut = ut / sqrt((q0 * q0 + q1 * q1) + q2 * q2);
     const double v1 = x1 * zt * ph.vscale_thermal;
     const double u = ut * v1 + un;
-    double nv = u + vcol + (quad(wcol, l0, n1) * quad(rs, l0, n2) - quad(wcol, l0, n2) * quad(rs, l0, n1));
+    double nv = u + vcol + (quad_next(wcol) * quad_prev(rs) - quad_prev(wcol) * quad_next(rs));
     if (sizeof(Real) == 4) nv = (double)(float)nv;  // what the velocity store keeps
     v = nv;
     o = o + v * dt * 0.5;
@@ -481,7 +493,7 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
                     bool inside = false;
                     unsigned reach = 0;
                     if (on) {
-                        fly<true>((pc & CURRENT) ? 1 : 1 + late, dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
+                        fly_flat((pc & CURRENT) ? 1 : 1 + late, dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
                         const float wx = (float)vx, wy = (float)vy, wz = (float)vz;
                         const float travel = sqrtf((wx * wx + wy * wy) + wz * wz) * wdt;
                         detect(all, ix, iy, iz, ox, oy, oz, travel, n_in, m_in, inside, reach);
@@ -534,7 +546,7 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
                     int phantom = pc & PHANTOM;
                     unpack_cell(pc, ix, iy, iz);
                     Real ox = s.o[0][i], oy = s.o[1][i], oz = s.o[2][i];
-                    fly<true>(1, dt, L, s.v[0][i], s.v[1][i], s.v[2][i], ix, iy, iz, ox, oy, oz);
+                    fly_flat(1, dt, L, s.v[0][i], s.v[1][i], s.v[2][i], ix, iy, iz, ox, oy, oz);
                     bool inside;
                     unsigned near;
                     detect(s.reach[i], ix, iy, iz, ox, oy, oz, 0.0f, n_in, m_in, inside, near);
@@ -592,10 +604,9 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
                 if (hit) {
                     // cpp/fluid_colloid_collision.cpp:40-42
                     c_lin = dump - v;
-                    const int n1 = k >= 2 ? 0 : k + 1, n2 = k == 0 ? 2 : k == 3 ? 1 : k - 1;
-                    c_ang = quad(rs, l0, n1) * quad(c_lin, l0, n2) - quad(rs, l0, n2) * quad(c_lin, l0, n1);
-                    const double bx = quad(o, l0, 0), by = quad(o, l0, 1), bz = quad(o, l0, 2);
-                    const double vx = quad(v, l0, 0), vy = quad(v, l0, 1), vz = quad(v, l0, 2);
+                    c_ang = quad_next(rs) * quad_prev(c_lin) - quad_prev(rs) * quad_next(c_lin);
+                    const double bx = quad<0>(o), by = quad<1>(o), bz = quad<2>(o);
+                    const double vx = quad<0>(v), vy = quad<1>(v), vz = quad<2>(v);
                     const double ax = (double)ix + bx, ay = (double)iy + by, az = (double)iz + bz;
                     // a later colloid that now contains it: the rest of the
                     // colloid loop is replayed serially
@@ -690,8 +701,8 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
             // cpp/update.cpp:34-46
             const double bk = w * ph.dt;
             const double sn = sin(bk), cs = cos(bk);
-            const double sbx = quad(sn, l0, 0), sby = quad(sn, l0, 1), sbz = quad(sn, l0, 2);
-            const double cbx = quad(cs, l0, 0), cby = quad(cs, l0, 1), cbz = quad(cs, l0, 2);
+            const double sbx = quad<0>(sn), sby = quad<1>(sn), sbz = quad<2>(sn);
+            const double cbx = quad<0>(cs), cby = quad<1>(cs), cbz = quad<2>(cs);
             double mx, my, mz;
             if (k == 0) { mx = cby * cbz; my = -cby * sbz; mz = sby; }
             else if (k == 1) { mx = sbx * sby * cbz + cbx * sbz; my = -sbx * sby * sbz + cbx * cbz; mz = -sbx * cby; }
@@ -728,10 +739,10 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
                 const int dm = pdiff(cc, s.cell0[c][k], L);
                 if (on && (dm > 1 || dm < -1)) tl_far = true;
                 const double md = img1(p - s.pos0[c][k], Ld);
-                const double m0 = quad(md, l0, 0), m1 = quad(md, l0, 1), m2 = quad(md, l0, 2);
+                const double m0 = quad<0>(md), m1 = quad<1>(md), m2 = quad<2>(md);
                 const double d2 = (m0 * m0 + m1 * m1) + m2 * m2;
                 const double wd = img1(p - s.posw[c][k], Ld);
-                const double w0 = quad(wd, l0, 0), w1 = quad(wd, l0, 1), w2 = quad(wd, l0, 2);
+                const double w0 = quad<0>(wd), w1 = quad<1>(wd), w2 = quad<2>(wd);
                 const double e2 = (w0 * w0 + w1 * w1) + w2 * w2;
                 if (on && d2 > 0.25 * MD_SKIN * MD_SKIN) md_far = true;
                 if (on && !last && d2 > ph.margin * ph.margin) marg = true;
@@ -787,7 +798,7 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
         unpack_cell(pc, ix, iy, iz);
         Real ox = now.ox, oy = now.oy, oz = now.oz;
         const Real vx = now.vx, vy = now.vy, vz = now.vz;
-        fly<true>(late, dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
+        fly_flat(late, dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
         f.cell[slot] = pack_cell(ix, iy, iz) | (pc & PHANTOM);
         f.ox[slot] = ox; f.oy[slot] = oy; f.oz[slot] = oz;
         f.vx[slot] = vx; f.vy[slot] = vy; f.vz[slot] = vz;
@@ -973,7 +984,7 @@ __global__ __launch_bounds__(COLLIDE_THREADS) void k_groups_redo(Phys ph, Dev d,
                     reaches_other(ph, d, R, (double)ix + (double)ox, (double)iy + (double)oy, (double)iz + (double)oz, vn, l - 1,
                                   [&](int g) { return d.redo[g] != 0; }))
                     escaped = true;
-                fly<true>(1, (Real)ph.dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
+                fly_flat(1, (Real)ph.dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
                 if (outside_tile_reach(R, ph.cap, slot, ix, iy, iz)) drift = true;
                 const double x = (double)ix + (double)ox, y = (double)iy + (double)oy, z = (double)iz + (double)oz;
                 int n_in = 0, gin = -1;

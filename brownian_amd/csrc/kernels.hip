@@ -1558,7 +1558,7 @@ __global__ __launch_bounds__(256) void k_classify(Phys ph, Dev d, Fluid<Real> f)
             });
             if (home < 0) {
                 // (a phantom that is inside no colloid ends being one)
-                fly<false>(ph.n_sub, (Real)ph.dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
+                fly(ph.n_sub, (Real)ph.dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
                 f.cell[slot] = pack_cell(ix, iy, iz);
                 f.ox[slot] = ox; f.oy[slot] = oy; f.oz[slot] = oz;
                 if (outside_tile_reach(R, ph.cap, slot, ix, iy, iz)) drift = true;
