@@ -21,7 +21,8 @@ size_t srd_lds_bytes(int ncell, int cap, bool fp64);
 size_t srd_static_lds();
 size_t srd_sur_lds();
 bool srd_needs_wrap(int L, int bmax);
-template <class Real> void launch_depart(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);
+template <class Real>
+void launch_depart(const Phys &, const Dev &, const Fluid<Real> &, const int2 *, int, bool, hipStream_t);
 template <class Real>
 void launch_srd(const Phys &, const Dev &, const Fluid<Real> &, const Fluid<Real> &, bool, bool, bool, size_t,
                 hipStream_t);
@@ -41,7 +42,7 @@ void launch_step_begin(const Phys &, const Dev &, hipStream_t, bool clear_lists 
 void launch_colloid(const Phys &, const Dev &, unsigned, hipStream_t);
 void launch_potential(const Phys &, const Dev &, int, hipStream_t);
 void launch_colloid_update(const Phys &, const Dev &, unsigned, const int2 *, int, hipStream_t);
-void launch_md_candidates(const Phys &, const Dev &, const int2 *, int, bool link, hipStream_t);
+void launch_md_candidates(const Phys &, const Dev &, const int2 *, int, hipStream_t);
 template <class Real> void launch_classify(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);
 // groups.hip
 template <class Real>
@@ -361,12 +362,9 @@ int enqueue_step(bw_ctx *c, int cur, int cb, bool final, bool groups, Prof *prof
         if (prof) prof->mark(st, BW_KERNEL_COLLOID);
     }
     launch_step_begin(ph, d0, st, col);  // with colloids it also clears the tile lists
-    if (col) {
-        launch_md_candidates(ph, d0, c->wgt, c->nwg, groups, st);
-        launch_tile_colloids(ph, d0, st, true);
-    }
+    if (col) launch_tile_colloids(ph, d0, st, true);
     if (prof) prof->mark(st, BW_KERNEL_COLLOID);
-    launch_depart<Real>(ph, d0, src, st);
+    launch_depart<Real>(ph, d0, src, c->wgt, col ? c->nwg : 0, groups, st);  // and the pair candidates
     if (prof) prof->mark(st, BW_KERNEL_DEPART);
     launch_srd<Real>(ph, d0, src, dst, col, false, c->block, c->srd_lds + (ph.surrogate ? srd_sur_lds() : 0), st);
     if (prof) prof->mark(st, BW_KERNEL_SRD);
@@ -1190,7 +1188,7 @@ BW_API int neighbour_list_md(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
     if (c->nc_total == 0) return BW_OK;
     Dev d = dev_for(c, c->cur);
-    launch_md_candidates(c->ph, d, c->wgt, c->nwg, false, c->st);
+    launch_md_candidates(c->ph, d, c->wgt, c->nwg, c->st);
     launch_colloid(c->ph, d, PH_MDLIST, c->st);
     return BW_OK;
 }
@@ -1222,10 +1220,10 @@ BW_API int rotation_mpcd(bw_ctx *c) {
     Dev d = dev_for(c, c->cur);
     launch_step_begin(c->ph, d, c->st);
     if (c->fp64) {
-        launch_depart<double>(c->ph, d, c->fl[c->cur].f64, c->st);
+        launch_depart<double>(c->ph, d, c->fl[c->cur].f64, nullptr, 0, false, c->st);
         launch_srd<double>(c->ph, d, c->fl[c->cur].f64, c->fl[1 - c->cur].f64, false, true, false, c->srd_lds, c->st);
     } else {
-        launch_depart<float>(c->ph, d, c->fl[c->cur].f32, c->st);
+        launch_depart<float>(c->ph, d, c->fl[c->cur].f32, nullptr, 0, false, c->st);
         launch_srd<float>(c->ph, d, c->fl[c->cur].f32, c->fl[1 - c->cur].f32, false, true, false, c->srd_lds, c->st);
     }
     c->cur ^= 1;

@@ -70,9 +70,8 @@ __global__ void k_colloid(Phys ph, Dev d, unsigned flags) {
 
 // one wave per colloid: every partner within cutoff + skin, ascending
 // link: also joins the groups of colloids closer than sqrt(link2)
-__global__ __launch_bounds__(256) void k_md_candidates(Phys ph, Dev d, const int2 *wgt, int link) {
+__device__ __forceinline__ void md_candidates(const Phys &ph, const Dev &d, const int2 wt, int link) {
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int2 wt = wgt[blockIdx.x];
     const Rep R = d.rep[wt.x];
     const int g = wt.y + w;
     if (g >= R.first_colloid + R.nc) return;
@@ -115,6 +114,9 @@ __global__ __launch_bounds__(256) void k_md_candidates(Phys ph, Dev d, const int
         }
         d.md_stale[wt.x] = 0;
     }
+}
+__global__ __launch_bounds__(256) void k_md_candidates(Phys ph, Dev d, const int2 *wgt) {
+    md_candidates(ph, d, wgt[blockIdx.x], 0);
 }
 
 // Per-tile colloid lists of the step, built colloid-first: the counters are
@@ -186,12 +188,22 @@ __device__ __forceinline__ int tile_delta(int tnew, int told, int nt) {
 // --------------------------------------------------------------- departure
 // For each particle of tile T, its tile on the SRD grid shifted by this step's
 // shift, as a direction 0..26; stable (array-order) lists per direction.
+// The first nwg blocks do the step's pair candidates instead (md_candidates,
+// which nothing before the substeps reads): bound by the waits of a few
+// workgroups, they were a launch of 5 us with 10 colloids and 32 us with 2400,
+// and run beside the tiles here (102 + 32 us, together 114 at 128^3; the bound
+// keeps the registers of the first from costing the tiles a wave per SIMD: 119).
 template <class Real>
-__global__ __launch_bounds__(DEPART_THREADS) void k_depart(Phys ph, Dev d, Fluid<Real> f) {
+__global__ __launch_bounds__(DEPART_THREADS, 8) void k_depart(Phys ph, Dev d, Fluid<Real> f, const int2 *wgt, int nwg, int link) {
+    static_assert(DEPART_THREADS == 256, "md_candidates: four waves");
+    if ((int)blockIdx.x < nwg) {
+        md_candidates(ph, d, ld_const(wgt + blockIdx.x), link);
+        return;
+    }
     constexpr int NW = DEPART_THREADS / 64, U = 4;  // waves; 64-particle groups whose loads fly together
     __shared__ unsigned char s_dir[MAX_CAP];
     __shared__ int s_cnt[NW][27], s_base[NW][27];
-    const int T = blockIdx.x;
+    const int T = (int)blockIdx.x - nwg;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     Rep R;
     TileGeo tg = tile_geo(d, T, R);
@@ -2315,8 +2327,8 @@ size_t srd_static_lds() { return sizeof(TileRun) + sizeof(NearColl) + 4 * TCL_CA
 size_t srd_sur_lds() { return SRD_SUR_LDS + 16; }
 
 template <class Real>
-void launch_depart(const Phys &ph, const Dev &d, const Fluid<Real> &f, hipStream_t st) {
-    LAUNCH(k_depart<Real>, ph.n_tiles, DEPART_THREADS, 0, st, ph, d, f);
+void launch_depart(const Phys &ph, const Dev &d, const Fluid<Real> &f, const int2 *wgt, int nwg, bool link, hipStream_t st) {
+    LAUNCH(k_depart<Real>, ph.n_tiles + nwg, DEPART_THREADS, 0, st, ph, d, f, wgt, nwg, (int)link);
 }
 template <class Real, bool C, bool M, bool B, bool W>
 static void srd_th(const Phys &ph, const Dev &d, const Fluid<Real> &src, const Fluid<Real> &dst, size_t lds,
@@ -2451,8 +2463,8 @@ void launch_colloid(const Phys &ph, const Dev &d, unsigned flags, hipStream_t st
 void launch_colloid_update(const Phys &ph, const Dev &d, unsigned flags, const int2 *wgt, int nwg, hipStream_t st) {
     LAUNCH(k_colloid_update, nwg, 256, 0, st, ph, d, flags, wgt);
 }
-void launch_md_candidates(const Phys &ph, const Dev &d, const int2 *wgt, int nwg, bool link, hipStream_t st) {
-    LAUNCH(k_md_candidates, nwg, 256, 0, st, ph, d, wgt, (int)link);
+void launch_md_candidates(const Phys &ph, const Dev &d, const int2 *wgt, int nwg, hipStream_t st) {
+    LAUNCH(k_md_candidates, nwg, 256, 0, st, ph, d, wgt);
 }
 void launch_tile_colloids(const Phys &ph, const Dev &d, hipStream_t st, bool cleared) {
     if (!cleared) LAUNCH(k_tile_lists_clear, (ph.n_tiles + 255) / 256, 256, 0, st, ph, d);
@@ -2519,7 +2531,8 @@ void launch_copy(const void *a, void *b, long long nbytes, hipStream_t st) {
 }
 
 #define INST(Real)                                                                                                 \
-    template void launch_depart<Real>(const Phys &, const Dev &, const Fluid<Real> &, hipStream_t);               \
+    template void launch_depart<Real>(const Phys &, const Dev &, const Fluid<Real> &, const int2 *, int, bool,    \
+                                      hipStream_t);                                                                \
     template void launch_srd<Real>(const Phys &, const Dev &, const Fluid<Real> &, const Fluid<Real> &, bool,    \
                                    bool, bool, size_t, hipStream_t);                                               \
     template void launch_stream<Real>(const Phys &, const Dev &, const Fluid<Real> &, bool, bool, bool, bool,     \
