@@ -2106,8 +2106,11 @@ __global__ void k_gather(Phys ph, Dev d, Fluid<Real> f, double *pos, double *vel
 // The colloid is driven by the surrogate in this step when surrogate mode is
 // on, the moments are valid and every feature lies in the training range;
 // otherwise it collides explicitly.  Resets the impulse accumulator.
-__global__ void k_features(Phys ph, Dev d, const int *colloid_rep) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+// Bound by the latency of its scattered reads: 32 lanes per colloid, a coarse
+// cell each (lanes 0..26) and a component of the colloid's own (27..31, then
+// 0..3 again); one thread per colloid was 84 us for 1227 colloids, this 8.7 us.
+__global__ __launch_bounds__(256) void k_features(Phys ph, Dev d, const int *colloid_rep) {
+    const int g = blockIdx.x * (256 / 32) + threadIdx.x / 32, o = threadIdx.x % 32;
     if (g >= ph.n_colloid_total) return;
     const int r = colloid_rep[g];
     const Rep R = d.rep[r];
@@ -2121,11 +2124,14 @@ __global__ void k_features(Phys ph, Dev d, const int *colloid_rep) {
         fo[k] = x;
         if (ph.surrogate && !(x >= d.sur_lo[k] && x <= d.sur_hi[k])) in = false;
     };
-    int c3[3];
-    for (int k = 0; k < 3; k++) c3[k] = coord_cell(mod1(d.cpos[3 * g + k] + d.shift[3 * r + k], Ld), L) / 2;
-    const double vcx = d.cvel[3 * g], vcy = d.cvel[3 * g + 1], vcz = d.cvel[3 * g + 2];
-    const double rho0 = 8.0 * (double)R.nf / ((double)L * L * L);
-    for (int o = 0; o < 27; o++) {
+    auto own = [&](int k) {  // k = 0..8
+        put(135 + k, (k < 3 ? d.cvel : k < 6 ? d.comega : d.cra)[3 * g + k % 3]);
+    };
+    if (o < 27) {
+        int c3[3];
+        for (int k = 0; k < 3; k++) c3[k] = coord_cell(mod1(d.cpos[3 * g + k] + d.shift[3 * r + k], Ld), L) / 2;
+        const double vcx = d.cvel[3 * g], vcy = d.cvel[3 * g + 1], vcz = d.cvel[3 * g + 2];
+        const double rho0 = 8.0 * (double)R.nf / ((double)L * L * L);
         const int qx = wrapi(c3[0] + o % 3 - 1, Lc), qy = wrapi(c3[1] + (o / 3) % 3 - 1, Lc),
                   qz = wrapi(c3[2] + o / 9 - 1, Lc);
         const float *mo = d.cmom + 5 * (R.first_coarse + qx + (long long)Lc * (qy + (long long)Lc * qz));
@@ -2139,15 +2145,16 @@ __global__ void k_features(Phys ph, Dev d, const int *colloid_rep) {
         put(5 * o, n / rho0);
         put(5 * o + 1, ux); put(5 * o + 2, uy); put(5 * o + 3, uz);
         put(5 * o + 4, t);
+    } else {
+        own(o - 27);
     }
-    for (int k = 0; k < 3; k++) {
-        put(135 + k, d.cvel[3 * g + k]);
-        put(138 + k, d.comega[3 * g + k]);
-        put(141 + k, d.cra[3 * g + k]);
+    if (o < 4) own(5 + o);
+    const unsigned out = (unsigned)(__ballot(!in) >> (threadIdx.x & 32));  // of this colloid's lanes
+    if (o == 0) {
+        d.cmode_prev[g] = d.cmode[g];
+        d.cmode[g] = out ? 0 : 1;
     }
-    d.cmode_prev[g] = d.cmode[g];
-    d.cmode[g] = in ? 1 : 0;
-    for (int k = 0; k < 6; k++) d.cimp[6 * g + k] = 0.0;
+    if (o < 6) d.cimp[6 * g + o] = 0.0;
 }
 
 // impulse of a surrogate-driven colloid over the coming step: mean + sd * xi,
@@ -2471,7 +2478,7 @@ void launch_tile_colloids(const Phys &ph, const Dev &d, hipStream_t st, bool cle
     if (ph.n_colloid_total > 0) LAUNCH(k_tile_colloids, ph.n_colloid_total, 256, 0, st, ph, d);
 }
 void launch_features(const Phys &ph, const Dev &d, const int *colloid_rep, hipStream_t st) {
-    LAUNCH(k_features, (ph.n_colloid_total + 63) / 64, 64, 0, st, ph, d, colloid_rep);
+    LAUNCH(k_features, (ph.n_colloid_total + 7) / 8, 256, 0, st, ph, d, colloid_rep);
 }
 void launch_sur_sample(const Phys &ph, const Dev &d, const int *colloid_rep, hipStream_t st) {
     LAUNCH(k_sur_sample, (ph.n_colloid_total + 63) / 64, 64, 0, st, ph, d, colloid_rep);
