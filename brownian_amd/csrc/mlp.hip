@@ -158,13 +158,17 @@ __global__ __launch_bounds__(256) void k_layer(const unsigned short *__restrict_
         Hb[(size_t)m * N + n] = f2bf(h);
     });
 }
-// the output layer: Y = X W + b
+// the output layer: Y = X W + b; rows not null: its first n rows without their
+// padding, n x MLP_OUT, in place of Y
 __global__ __launch_bounds__(256) void k_layer_out(const unsigned short *__restrict__ X, const unsigned short *__restrict__ W,
-                                                   const float *__restrict__ bias, int M, float *__restrict__ Y) {
+                                                   const float *__restrict__ bias, int M, float *__restrict__ Y,
+                                                   float *__restrict__ rows, int n_rows) {
     __shared__ __align__(16) unsigned short s[2 * GEMM_B * GEMM_KS];
     const f32x16 acc = gemm_block<0, 0>(X, W, M, MLP_OUTP, MLP_H, MLP_H, MLP_OUTP, blockIdx.x * GEMM_B, 0, s);
-    gemm_elements(acc, M, MLP_OUTP, blockIdx.x * GEMM_B, 0,
-                  [&](int m, int n, float v) { Y[(size_t)m * MLP_OUTP + n] = v + bias[n]; });
+    gemm_elements(acc, M, MLP_OUTP, blockIdx.x * GEMM_B, 0, [&](int m, int n, float v) {
+        if (!rows) Y[(size_t)m * MLP_OUTP + n] = v + bias[n];
+        else if (m < n_rows && n < MLP_OUT) rows[(size_t)m * MLP_OUT + n] = v + bias[n];
+    });
 }
 
 __global__ void k_to_bf16(const float *__restrict__ x, unsigned short *__restrict__ y, long long n) {
@@ -353,14 +357,6 @@ constexpr int NOALLOC_ROWS = 1024;
 constexpr size_t NOALLOC_ROW_BYTES = (size_t)MLP_INP * 2 + (size_t)MLP_OUTP * 4 + 3 * ((size_t)MLP_H * 2);
 static __device__ __align__(256) unsigned char scratch[NOALLOC_ROWS * NOALLOC_ROW_BYTES];
 
-// rows [0, n) of the padded output (stride MLP_OUTP) -> n x MLP_OUT
-__global__ void k_mlp_rows(const float *__restrict__ y, int n, float *__restrict__ out) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n * MLP_OUT) return;
-    const int i = e / MLP_OUT, k = e - i * MLP_OUT;
-    out[e] = y[(size_t)i * MLP_OUTP + k];
-}
-
 }  // namespace bw
 
 using namespace bw;
@@ -382,6 +378,7 @@ struct bw_mlp {
     MlpBuf tb;  // training / host-call activations
     unsigned char *scratch = nullptr;  // device address of the scratch array on the network's GPU
     float *xin = nullptr, *tin = nullptr, *yout = nullptr;  // a host call's rows (grown as needed)
+    float *ypin = nullptr;    // outputs of up to PINNED_ROWS rows, in pinned host memory
     long long xin_rows = 0;
     // data set on the device, and the rows' losses
     float *dX = nullptr, *dT = nullptr, *dloss = nullptr;
@@ -539,11 +536,11 @@ void forward_hidden(bw_mlp *m, MlpBuf &B, const float *x, const int *idx, int n,
         hipLaunchKernelGGL(k_layer, dim3(back_blocks(n_pad, m->N[l])), dim3(256), 0, st, l == 0 ? B.Xb : B.Hb[l - 1], m->Wb[l],
                            m->b[l], n_pad, m->N[l], m->K[l], train ? B.Z[l] : nullptr, B.Hb[l]);
 }
-// outputs of rows [0, n) in B.Y (n_pad x 32)
-void forward(bw_mlp *m, MlpBuf &B, const float *x, const int *idx, int n, int n_pad, hipStream_t st) {
+// outputs of rows [0, n) in B.Y (n_pad x 32), or in rows (n x 12) if that is not null
+void forward(bw_mlp *m, MlpBuf &B, const float *x, const int *idx, int n, int n_pad, hipStream_t st, float *rows = nullptr) {
     forward_hidden(m, B, x, idx, n, n_pad, false, st);
     hipLaunchKernelGGL(k_layer_out, dim3((n_pad + GEMM_B - 1) / GEMM_B), dim3(256), 0, st, B.Hb[2], m->Wb[3], m->b[3], n_pad,
-                       B.Y);
+                       B.Y, rows, n);
 }
 
 ParamTable param_table(const bw_mlp *m) {
@@ -664,6 +661,7 @@ BW_API int bw_mlp_destroy(bw_mlp *m) {
     mlp_buf_free(m->tb);
     for (void *q : {(void *)m->dX, (void *)m->dT, (void *)m->didx, (void *)m->dloss, (void *)m->xin, (void *)m->tin, (void *)m->yout})
         if (q) hipFree(q);
+    if (m->ypin) hipHostFree(m->ypin);
     if (m->st) hipStreamDestroy(m->st);
     delete m;
     return BW_OK;
@@ -707,17 +705,26 @@ BW_API int bw_mlp_set_normalisation(bw_mlp *m, const float *x_mean, const float 
     return BW_OK;
 }
 
+constexpr int PINNED_ROWS = 1024;
 // y (n x 12): standardised mean (6) and log-variance (6) for host features x (n x 144)
 BW_API int bw_mlp_forward(bw_mlp *m, const float *x, int n, float *y) {
     if (!m || !x || !y || n < 1) return BW_ERR_ARG;
     int n_pad = (n + 31) / 32 * 32, rc;
     if ((rc = ensure_batch(m, n_pad, false)) || (rc = ensure_rows(m, n))) return rc;
-    MCHK(m, hipMemcpyAsync(m->xin, x, sizeof(float) * (size_t)n * MLP_IN, hipMemcpyHostToDevice, m->st));
-    forward(m, m->tb, m->xin, nullptr, n, n_pad, m->st);
-    hipLaunchKernelGGL(k_mlp_rows, dim3((unsigned)(((long long)n * MLP_OUT + 255) / 256)), dim3(256), 0, m->st, m->tb.Y, n,
-                       m->yout);
-    MCHK(m, hipMemcpyAsync(y, m->yout, sizeof(float) * (size_t)n * MLP_OUT, hipMemcpyDeviceToHost, m->st));
+    // (not copies queued on the stream: those of pageable memory take longer,
+    // 902 rows 109 us in all against 83; here 75)
+    MCHK(m, hipMemcpy(m->xin, x, sizeof(float) * (size_t)n * MLP_IN, hipMemcpyHostToDevice));
+    // few rows are written to pinned host memory by the output layer itself (a
+    // copy of them would take 10 to 20 us)
+    if (n <= PINNED_ROWS && !m->ypin && hipHostMalloc((void **)&m->ypin, sizeof(float) * PINNED_ROWS * MLP_OUT, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        m->ypin = nullptr;
+    }
+    const bool pinned = n <= PINNED_ROWS && m->ypin;
+    forward(m, m->tb, m->xin, nullptr, n, n_pad, m->st, pinned ? m->ypin : m->yout);
     MCHK(m, hipStreamSynchronize(m->st));
+    if (pinned) memcpy(y, m->ypin, sizeof(float) * (size_t)n * MLP_OUT);
+    else MCHK(m, hipMemcpy(y, m->yout, sizeof(float) * (size_t)n * MLP_OUT, hipMemcpyDeviceToHost));
     return BW_OK;
 }
 
@@ -732,8 +739,7 @@ BW_API int bw_mlp_forward_noalloc(bw_mlp *m, const float *x, int n, float *y) {
     if (!m->scratch) return mfail(m, BW_ERR_STATE, "bw_mlp_forward_noalloc: no scratch address");
     const int n_pad = (n + 31) / 32 * 32;
     MlpBuf B = scratch_buf(m->scratch, n_pad);
-    forward(m, B, x, nullptr, n, n_pad, m->st);
-    hipLaunchKernelGGL(k_mlp_rows, dim3((n * MLP_OUT + 255) / 256), dim3(256), 0, m->st, B.Y, n, y);
+    forward(m, B, x, nullptr, n, n_pad, m->st, y);
     MCHK(m, hipGetLastError());
     MCHK(m, hipStreamSynchronize(m->st));
     return BW_OK;
