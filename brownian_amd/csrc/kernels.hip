@@ -2,19 +2,24 @@
 //
 // Fused MPCD step (one replica or many, one launch per kernel for all):
 //   k_step_begin       step counter, grid shift of this step               (1 WG)
-//   k_md_candidates    colloid pair candidates (cutoff + skin)              (1 wave / colloid)
-//   k_tile_colloids    per tile: colloids that can touch it this step        (1 WG / tile)
-//   k_depart           per tile: each particle's tile on the new shifted
-//                      grid, stable departure lists per direction           (1 WG / tile)
-//   k_srd              per tile: gather from 27 neighbour lists, LDS
-//                      counting sort by shifted cell, FP64 per-cell sums,
-//                      rotation + thermostat, run() shell counts             (1 WG / tile)
-//   n_sub x { k_stream          per tile: run() kick (first substep), streaming,
-//                                detection through LDS stencil masks
-//             k_collide         1 wave / colloid: pair list, reflections;
-//                                last WG of a replica: serial replays
+//   k_tile_colloids    per tile: colloids that can touch it this step        (1 WG / colloid)
+//   k_depart           colloid pair candidates, cutoff + skin (1 wave /
+//                      colloid); per tile: each particle's tile on the new
+//                      shifted grid, stable departure lists per direction    (1 WG / tile)
+//   k_srd              per tile: gather from 27 neighbour lists, per-cell
+//                      sums, rotation + thermostat, run() shell counts,
+//                      flight of the particles far from every colloid        (1 WG / tile)
+// then the substeps, either by colloid groups (groups.hip, the usual way):
+//   k_classify         run() kick, first streaming, particles that may reach
+//                      a colloid into its bucket (the others fly the step)   (near chunks)
+//   k_group_lists, k_groups, k_groups_redo
+// or kernel by kernel (BW_STREAM_PER_SUBSTEP, boxes whose colloids form large
+// groups):
+//   n_sub x { k_stream / k_stream_near  streaming, detection
+//             k_collide         1 wave / colloid: pair list, reflections
+//             k_serial          1 WG / replica: serial replays
 //             k_colloid_update  1 wave / colloid: collision impulse, activity,
-//                                WCA force, velocity, [kick], position }
+//                               WCA force, velocity, [kick], position }
 #include "bw_device.h"
 #include "collide.h"
 

@@ -43,7 +43,9 @@ extern "C" {
 #define BW_FLAG_ZERO_VARIANCE 0x80u    /* thermostat on a cell with zero relative KE      */
 #define BW_FLAG_NEIGH_OVERFLOW 0x100u  /* neigh_fl capacity exceeded                      */
 #define BW_FLAG_MARGIN 0x200u          /* a colloid moved beyond the blocked-streaming margin
-                                          within one step (use BW_STREAM_PER_SUBSTEP)    */
+                                          within one step, or a reflected particle may have
+                                          reached one outside its group (use
+                                          BW_STREAM_PER_SUBSTEP)                         */
 
 enum bw_precision { BW_FP32 = 0, BW_FP64 = 1 };
 enum bw_vel_law { BW_VEL_REFERENCE = 0, BW_VEL_MAXWELL = 1 };
