@@ -335,11 +335,9 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
     int par = 0, n_events = 0, n_sel = 0, n_se = 0;
     int opened = 0;            // the window's first substep
     const Real dt = (Real)ph.dt;
-    // FP32 positions are taken from the first colloid's cell; a group that may
-    // stretch over half the box takes their differences modulo L
+    // FP32 positions are taken from the first colloid's cell
     const int o0 = d.ccell[3 * s.g[0]], o1 = d.ccell[3 * s.g[0] + 1], o2 = d.ccell[3 * s.g[0] + 2];
     const double origin[3] = {(double)o0, (double)o1, (double)o2};
-    const bool wrap = 0.5 * Ld < C * sqrt(ph.link2) + 4.0;
     const float Lf = (float)L, iLf = 1.0f / Lf;
     for (int i = tid; i < C * 3; i += TH) {
         const int c = i / 3, k = i - 3 * c, g = s.g[c];
@@ -377,6 +375,17 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
     h += d.grp_hot[s.g[0]];  // the group's working copies
     int *slots = d.grp_slot + d.grp_hot[s.g[0]];
     sync();
+    // A particle's position from the origin lies in [-L/2, L/2 + 1), so its
+    // distance to a colloid at b is taken right without the wrap modulo L as
+    // long as |b| plus that distance stays below L/2 - 1 along every axis:
+    // distances up to `room` (the group's own extent: fast particles link
+    // colloids farther apart than link2)
+    float extent = 0.0f;
+    for (int c = 0; c < C; c++) {
+        const float4 b = s.rel[0][c];
+        extent = fmaxf(extent, fmaxf(fabsf(b.x), fmaxf(fabsf(b.y), fabsf(b.z))));
+    }
+    const float room = 0.5f * Lf - 1.0f - (extent + (float)ph.margin + 1e-2f);
     unsigned all = 0;  // the explicitly colliding colloids
     for (int c = 0; c < C; c++)
         if (!s.sur[c]) all |= 1u << c;
@@ -403,11 +412,11 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
                 const int c = __ffs(m) - 1;
                 const float4 b = s.rel[par][c];
                 float ax = px - b.x, ay = py - b.y, az = pz - b.z;
-                if (wrap) {
+                const float rs = open ? r0 + b.w : rd;
+                if (!(rs <= room)) {
                     ax -= Lf * rintf(ax * iLf); ay -= Lf * rintf(ay * iLf); az -= Lf * rintf(az * iLf);
                 }
                 const float q2 = (ax * ax + ay * ay) + az * az;
-                const float rs = open ? r0 + b.w : rd;
                 if (q2 > rs * rs) continue;
                 reach |= 1u << c;
                 if (q2 > rd * rd) continue;
