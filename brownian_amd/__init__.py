@@ -357,6 +357,12 @@ class System:
         self._chk(self.lib.bw_get_surrogate_shells(self.h, replica, _ptr(cnt, _ip), _ptr(sums)))
         return cnt, sums
 
+    def step_paths(self) -> dict:
+        """Fused steps so far by the way their substeps were taken (same results)."""
+        o = (C.c_longlong * 3)()
+        self._chk(self.lib.bw_step_paths(self.h, o))
+        return dict(groups=o[0], again=o[1], per_substep=o[2])
+
     def near_particles(self, replica=0) -> int:
         n = C.c_longlong(0)
         self._chk(self.lib.bw_near_particles(self.h, replica, C.byref(n)))

@@ -39,6 +39,7 @@ template <class Real> void launch_audit(const Phys &, const Dev &, const Fluid<R
 template <class Real>
 void launch_gather(const Phys &, const Dev &, const Fluid<Real> &, double *, double *, int *, int, int, hipStream_t);
 void launch_step_begin(const Phys &, const Dev &, hipStream_t, bool clear_lists = false);
+void launch_restore(const Phys &, const Dev &, hipStream_t);
 void launch_colloid(const Phys &, const Dev &, unsigned, hipStream_t);
 void launch_potential(const Phys &, const Dev &, int, hipStream_t);
 void launch_colloid_update(const Phys &, const Dev &, unsigned, const int2 *, int, hipStream_t);
@@ -88,6 +89,12 @@ struct ReplicaHost {
     long long obs_step0 = 0;
 };
 
+// a step by groups that was launched and not yet seen to be finished
+struct QueuedStep {
+    int cur, cb;           // the buffers it starts from (cb after its prologue)
+    bool final, prologue;
+};
+
 struct FluidAlloc {
     void *base = nullptr;
     Fluid<float> f32;
@@ -135,14 +142,18 @@ struct bw_ctx {
     MlpBuf mbuf;                    // its activations for the step's inference
     hipGraphExec_t graphs[2][2][2][2] = {};  // [cur][cb][final][by groups]
     // colloid groups: the step may run by groups; working copies of their
-    // particles; what k_groups_redo had to take (host memory that the device
-    // writes), what of it has been looked at and after how many steps, and the
-    // steps still to run per substep because of it
+    // particles; the number of a stopped step (host memory that the device
+    // writes, 0: none); the steps launched and not yet looked at (settle)
     bool groups = false;
     HotPart<float> *hot32 = nullptr;
     HotPart<double> *hot64 = nullptr;
-    int *redo_stat = nullptr;
-    int redo_seen = 0, group_steps = 0, skip_groups = 0;
+    long long *halt_step = nullptr;
+    std::vector<QueuedStep> queued;
+    // steps finished by groups since one was stopped; steps to take kernel by
+    // kernel before the next try, and how many the last time; that try follows
+    int good = 0, skip = 0, backoff = 0;
+    bool trying = false;
+    long long path_steps[3] = {0, 0, 0};  // by groups, stopped and taken again, kernel by kernel
 };
 
 namespace {
@@ -342,9 +353,10 @@ struct Prof {
 // of this step done (by the previous step's last colloid update or the
 // prologue).  `final`: the last colloid update stops after
 // update_velocity_colloid.  groups: the substeps by colloid groups (same
-// results) instead of kernel by kernel over all colloids.
+// results) instead of kernel by kernel over all colloids.  again: a stopped
+// step, whose surrogate inputs stand.
 template <class Real>
-int enqueue_step(bw_ctx *c, int cur, int cb, bool final, bool groups, Prof *prof) {
+int enqueue_step(bw_ctx *c, int cur, int cb, bool final, bool groups, Prof *prof, bool again = false) {
     hipStream_t st = c->st;
     Phys ph = c->ph;
     ph.groups = groups;
@@ -352,7 +364,7 @@ int enqueue_step(bw_ctx *c, int cur, int cb, bool final, bool groups, Prof *prof
     Fluid<Real> &src = fluid_of<Real>(c, cur), &dst = fluid_of<Real>(c, 1 - cur);
     Dev d0 = dev_at(c, cur, cb);
     if (prof) prof->mark(st, BW_KERNEL_OTHER);
-    if (col && ph.moments) {
+    if (col && ph.moments && !again) {
         // surrogate inputs from the last rotation pass (its shift is still current)
         launch_features(ph, d0, c->colloid_rep, st);
         if (ph.surrogate) {
@@ -371,6 +383,7 @@ int enqueue_step(bw_ctx *c, int cur, int cb, bool final, bool groups, Prof *prof
     if (col && ph.surrogate) launch_sur_shell_kick<Real>(ph, dev_at(c, 1 - cur, cb), dst, st);
     if (groups) {
         Dev d1 = dev_at(c, 1 - cur, cb);
+        d1.status++;
         launch_classify<Real>(ph, d1, dst, st);
         if (prof) prof->mark(st, BW_KERNEL_STREAM);
         launch_groups<Real>(ph, d1, dst, hot_of<Real>(c), final, st);
@@ -403,7 +416,9 @@ int enqueue_step(bw_ctx *c, int cur, int cb, bool final, bool groups, Prof *prof
 template <class Real>
 void enqueue_prologue(bw_ctx *c) {
     if (c->nc_total == 0) return;
-    launch_colloid(c->ph, dev_for(c, c->cur), PH_KICK | PH_OLDF | PH_POS, c->st);
+    Phys ph = c->ph;
+    ph.groups = c->groups;  // (not behind a stopped step)
+    launch_colloid(ph, dev_for(c, c->cur), PH_KICK | PH_OLDF | PH_POS, c->st);
     c->cb ^= 1;
 }
 
@@ -418,25 +433,6 @@ int build_graph(bw_ctx *c, int cur, int cb, int final, int groups) {
     return BW_OK;
 }
 
-// Whether the next step runs by groups.  What k_groups_redo takes is slow there
-// (its one workgroup needs about half of what the per-substep launches of a
-// whole step need, more with many colloids): where more than a third of the
-// steps redid some, or one redid far more colloids than a group holds, the next
-// steps run per substep, with the same results.
-bool by_groups(bw_ctx *c) {
-    if (!c->groups) return false;
-    volatile int *redone = c->redo_stat;
-    if (c->skip_groups == 0 && (++c->group_steps >= 20 || redone[1] > 2 * GROUP_MAX)) {
-        if (redone[0] - c->redo_seen > c->group_steps / 3 || redone[1] > 2 * GROUP_MAX) c->skip_groups = 200;
-        c->redo_seen = redone[0];
-        redone[1] = 0;
-        c->group_steps = 0;
-    }
-    if (c->skip_groups == 0) return true;
-    c->skip_groups--;
-    return false;
-}
-
 // colloid buffer after one step from buffer cb: one flip per update_pos_md,
 // or one in all by groups
 int cb_after(const bw_ctx *c, int cb, bool final, bool groups) {
@@ -446,44 +442,137 @@ int cb_after(const bw_ctx *c, int cb, bool final, bool groups) {
     return cb ^ (npos & 1);
 }
 
+// Whether the next step runs by groups.  A stopped step costs 0.3 ms beyond
+// the step kernel by kernel (64^3: 0.84 ms, by groups 0.36), so two steps by
+// groups pay for it.  Where steps are stopped one after another (a cluster
+// beyond a group's lists) the next ones run kernel by kernel, 1, 3, 7, ... up
+// to MAX_BACKOFF between tries (64^3, 144 colloids in one cluster, 100 steps:
+// 0.86 ms a step).
+constexpr int MAX_BACKOFF = 511;
+constexpr int GOOD_STEPS = 2;
+bool by_groups(const bw_ctx *c) { return c->groups && c->skip == 0; }
+
+// one step with the prologue it needs, by groups or kernel by kernel
 template <class Real>
-int do_steps(bw_ctx *c, int n) {
+int one_step(bw_ctx *c, bool final, Prof *prof) {
+    const bool grp = by_groups(c), prologue = c->pending_prologue;
+    if (prologue) enqueue_prologue<Real>(c);
+    c->pending_prologue = false;
+    const QueuedStep q{c->cur, c->cb, final, prologue};
+    if (prof) {
+        c->cb = enqueue_step<Real>(c, c->cur, c->cb, final, grp, prof);
+    } else {
+        hipGraphExec_t &graph = c->graphs[c->cur][c->cb][final][grp];
+        if (!graph)
+            if (const int rc = build_graph<Real>(c, c->cur, c->cb, final, grp)) return rc;
+        HIPCHK(c, hipGraphLaunch(graph, c->st));
+        c->cb = cb_after(c, c->cb, final, grp);
+    }
+    c->cur ^= 1;
+    c->steps_done++;
+    c->pending_prologue = final;
+    if (grp) {
+        c->queued.push_back(q);
+    } else {
+        c->path_steps[2]++;
+        if (c->skip > 0) c->trying = --c->skip == 0;
+    }
+    return BW_OK;
+}
+
+// Waits for the launched steps by groups; a stopped one is taken again kernel
+// by kernel, and those behind it, which did nothing, in the usual way.
+// Everything that reads or changes the state comes through here first.
+// idle: the stream has been waited for.
+template <class Real>
+int settle_impl(bw_ctx *c, bool idle) {
+    std::vector<QueuedStep> again;  // the first is next
+    for (;;) {
+        if (!c->queued.empty()) {
+            if (!idle) HIPCHK(c, hipStreamSynchronize(c->st));
+            idle = false;
+            c->trying = false;
+            const long long halted = *(volatile long long *)c->halt_step;
+            const size_t n = c->queued.size(), i = halted ? (size_t)(halted - (c->steps_done - (long long)n) - 1) : n;
+            if (i > n || (halted && i == n)) return fail(c, BW_ERR_STATE, "a stopped step that was not launched");
+            c->good = (int)std::min<long long>((long long)c->good + (long long)i, INT_MAX);
+            c->path_steps[0] += (long long)i;
+            if (i < n) {
+                const QueuedStep q = c->queued[i];
+                again.insert(again.begin(), c->queued.begin() + i + 1, c->queued.end());
+                c->queued.clear();
+                *(volatile long long *)c->halt_step = 0;
+                c->backoff = c->good >= GOOD_STEPS ? 0 : std::min(MAX_BACKOFF, 2 * c->backoff + 1);
+                c->skip = c->backoff;
+                c->good = 0;
+                c->path_steps[1]++;
+                c->steps_done -= (long long)(n - i);
+                c->cur = q.cur;
+                launch_restore(c->ph, dev_at(c, q.cur, q.cb), c->st);
+                c->cb = enqueue_step<Real>(c, q.cur, q.cb, q.final, false, nullptr, true);
+                HIPCHK(c, hipGetLastError());
+                c->cur ^= 1;
+                c->steps_done++;
+                c->pending_prologue = q.final;
+            }
+            c->queued.clear();
+        }
+        if (again.empty()) return BW_OK;
+        // a few at a time, so that few are in vain behind the next stopped one
+        size_t m = 0;
+        while (m < again.size() && m < 8 && (by_groups(c) || c->queued.empty())) {
+            c->pending_prologue = again[m].prologue;
+            if (const int rc = one_step<Real>(c, again[m].final, nullptr)) return rc;
+            m++;
+        }
+        again.erase(again.begin(), again.begin() + m);
+    }
+}
+int settle(bw_ctx *c, bool idle = false) {
+    if (!c || c->queued.empty()) return BW_OK;
+    return c->fp64 ? settle_impl<double>(c, idle) : settle_impl<float>(c, idle);
+}
+// settle for calls that read the state and wait for the stream themselves
+// (read): behind the launched steps at once, and again in the rare case that
+// one of them was stopped
+template <class F>
+int read_settled(bw_ctx *c, F &&read) {
+    int rc = read();
+    if (c->queued.empty()) return rc;
+    const bool stopped = *(volatile long long *)c->halt_step != 0;
+    const int rs = settle(c, rc == BW_OK);
+    return rs ? rs : stopped ? read() : rc;
+}
+#define SETTLE(c)                                    \
+    do {                                             \
+        if (const int rc_ = settle(c)) return rc_;   \
+    } while (0)
+
+template <class Real>
+int do_steps(bw_ctx *c, int n, Prof *prof) {
     if (n <= 0) return BW_OK;
     int rc = sync_injected(c);
     if (rc) return rc;
-    if (c->pending_prologue) enqueue_prologue<Real>(c);
-    c->pending_prologue = false;
     for (int s = 0; s < n; s++) {
-        int fin = (s == n - 1) ? 1 : 0;
-        const int grp = by_groups(c) ? 1 : 0;
-        if (!c->graphs[c->cur][c->cb][fin][grp])
-            if ((rc = build_graph<Real>(c, c->cur, c->cb, fin, grp))) return rc;
-        HIPCHK(c, hipGraphLaunch(c->graphs[c->cur][c->cb][fin][grp], c->st));
-        c->cb = cb_after(c, c->cb, fin != 0, grp != 0);
-        c->cur ^= 1;
-        c->steps_done++;
+        if ((rc = one_step<Real>(c, s == n - 1, prof))) return rc;
+        // a try after stopped steps is looked at before more follow it; and
+        // the list of steps stays bounded
+        if ((c->trying && !c->queued.empty()) || c->queued.size() >= 65536) {
+            if ((rc = settle(c))) return rc;
+        }
     }
-    c->pending_prologue = true;
     c->substep = 0;
     return BW_OK;
 }
 
 template <class Real>
 int do_profile(bw_ctx *c, int n, double *ms, int *launches) {
-    int rc = sync_injected(c);
+    int rc = settle(c);
     if (rc) return rc;
     for (int k = 0; k < BW_KERNEL_COUNT; k++) { ms[k] = 0; if (launches) launches[k] = 0; }
     Prof prof;
-    for (int s = 0; s < n; s++) {
-        if (c->pending_prologue) enqueue_prologue<Real>(c);
-        c->pending_prologue = false;
-        c->cb = enqueue_step<Real>(c, c->cur, c->cb, s == n - 1, by_groups(c), &prof);
-        c->cur ^= 1;
-        c->steps_done++;
-    }
+    if ((rc = do_steps<Real>(c, n, &prof))) return rc;
     prof.mark(c->st, BW_KERNEL_OTHER);
-    c->pending_prologue = true;
-    c->substep = 0;
     HIPCHK(c, hipStreamSynchronize(c->st));
     for (size_t i = 0; i + 1 < prof.ev.size(); i++) {
         float t = 0;
@@ -493,7 +582,7 @@ int do_profile(bw_ctx *c, int n, double *ms, int *launches) {
         if (launches) launches[fam] += 1;
     }
     for (auto e : prof.ev) hipEventDestroy(e);
-    return BW_OK;
+    return settle(c);
 }
 
 // ------------------------------------------------------------------ create
@@ -537,14 +626,12 @@ int setup_groups(bw_ctx *c) {
         (rc = dalloc(c, &d.grp_mem, NC)) || (rc = dalloc(c, &d.grp_big, NC)) || (rc = dalloc(c, &d.grp_small, NC)) ||
         (rc = dalloc(c, &d.grp_cnt, 2)) || (rc = dalloc(c, &d.hot_cnt, NC)) ||
         (rc = dalloc(c, &d.hot_ent, NH)) || (rc = dalloc(c, &d.ovl_cnt, 1)) || (rc = dalloc(c, &d.ovl_g, OVL_CAP)) ||
-        (rc = dalloc(c, &d.ovl_slot, OVL_CAP)) || (rc = dalloc(c, &d.redo, NC)) || (rc = dalloc(c, &d.redo_list, NC)) ||
-        (rc = dalloc(c, &d.redo_cnt, c->n_rep)) ||
-        (rc = dalloc(c, &d.redo_mark, 3)))
+        (rc = dalloc(c, &d.ovl_slot, OVL_CAP)) || (rc = dalloc(c, &d.halt, 1)) || (rc = dalloc(c, &d.save, SAVE_WORDS * NC)))
         return rc;
     if ((rc = c->fp64 ? dalloc(c, &c->hot64, NH) : dalloc(c, &c->hot32, NH))) return rc;
-    HIPCHK(c, hipHostMalloc((void **)&c->redo_stat, 2 * sizeof(int), hipHostMallocMapped));
-    c->redo_stat[0] = c->redo_stat[1] = 0;
-    HIPCHK(c, hipHostGetDevicePointer((void **)&d.redo_stat, c->redo_stat, 0));
+    HIPCHK(c, hipHostMalloc((void **)&c->halt_step, sizeof(long long), hipHostMallocMapped));
+    *c->halt_step = 0;
+    HIPCHK(c, hipHostGetDevicePointer((void **)&d.halt_step, c->halt_step, 0));
     c->groups = true;
     return BW_OK;
 }
@@ -787,7 +874,7 @@ int create_impl(const bw_params *ps, int n_rep, bw_ctx **out) {
         (rc = dalloc(c, &d.cont_cnt, n_rep)) || (rc = dalloc(c, &d.cont_slot, (size_t)n_rep * CONT_CAP)) ||
         (rc = dalloc(c, &d.cont_from, (size_t)n_rep * CONT_CAP)) ||
         (rc = dalloc(c, &d.cont_dump, (size_t)n_rep * CONT_CAP * 3)) ||
-        (rc = dalloc(c, &d.status, 1)) || (rc = dalloc(c, &d.step, 1)) ||
+        (rc = dalloc(c, &d.status, 2)) || (rc = dalloc(c, &d.step, 1)) ||
         (rc = dalloc(c, &d.shift, 3 * n_rep)) || (rc = dalloc(c, &d.audit_partial, (size_t)tiles * 8))) {
         *out = c;
         return rc;
@@ -978,7 +1065,7 @@ BW_API int bw_ctx_destroy(bw_ctx *c) {
     if (c->st) hipStreamSynchronize(c->st);
     destroy_graphs(c);
     for (void *q : c->allocs) hipFree(q);
-    if (c->redo_stat) hipHostFree(c->redo_stat);
+    if (c->halt_step) hipHostFree(c->halt_step);
     mlp_buf_free(c->mbuf);
     const void *inj[] = {c->dv.inj_shift, c->dv.inj_axes, c->dv.inj_off, c->dv.inj_pid, c->dv.inj_val,
                          c->dv.sur_lo, c->dv.sur_hi};
@@ -998,14 +1085,17 @@ BW_API int bw_replica_info(bw_ctx *c, int r, int *o) {
     return BW_OK;
 }
 BW_API int bw_sync(bw_ctx *c) {
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     return BW_OK;
 }
 BW_API int bw_status(bw_ctx *c, unsigned *flags) {
-    unsigned s = 0;
+    SETTLE(c);
+    unsigned w[2] = {0, 0};
     HIPCHK(c, hipStreamSynchronize(c->st));
-    HIPCHK(c, hipMemcpy(&s, c->dv.status, sizeof(unsigned), hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemsetAsync(c->dv.status, 0, sizeof(unsigned), c->st));
+    HIPCHK(c, hipMemcpy(w, c->dv.status, sizeof w, hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemsetAsync(c->dv.status, 0, sizeof w, c->st));
+    const unsigned s = w[0] | w[1];
     if (flags) *flags = s;
     if (s) {
         char buf[96];
@@ -1023,7 +1113,15 @@ BW_API int initialize(bw_ctx *c) {
     // ordered on the context's stream before any later launch
     for (int b = 0; b < 2; b++) HIPCHK(c, hipMemsetAsync(c->counts[b], 0, sizeof(int) * c->ph.n_tiles, c->st));
     HIPCHK(c, hipMemsetAsync(c->dv.step, 0, sizeof(long long), c->st));
-    HIPCHK(c, hipMemsetAsync(c->dv.status, 0, sizeof(unsigned), c->st));
+    HIPCHK(c, hipMemsetAsync(c->dv.status, 0, 2 * sizeof(unsigned), c->st));
+    // of earlier steps nothing counts any more, also not that one was stopped
+    c->queued.clear();
+    c->good = c->skip = c->backoff = 0;
+    c->trying = false;
+    if (c->groups) {
+        *(volatile long long *)c->halt_step = 0;
+        HIPCHK(c, hipMemsetAsync(c->dv.halt, 0, sizeof(int), c->st));
+    }
     size_t NC = std::max(c->nc_total, 1);
     double *arrs[] = {c->cposb[0], c->cposb[1], c->dv.cvel, c->dv.comega, c->dv.cf, c->dv.coldf,
                       c->dv.cra, c->dv.cdisp, c->dv.cdv, c->dv.cdw};
@@ -1117,7 +1215,7 @@ int init_fluid_device(bw_ctx *c) {
     if (!list.empty()) HIPCHK(c, hipMemcpy(dlist, list.data(), sizeof(int) * list.size(), hipMemcpyHostToDevice));
     InitBins b{dG, dfirst, dstart, dlist, c->cposb[c->cb]};
     Dev d = dev_for(c, c->cur);
-    HIPCHK(c, hipMemsetAsync(c->dv.status, 0, sizeof(unsigned), c->st));
+    HIPCHK(c, hipMemsetAsync(c->dv.status, 0, 2 * sizeof(unsigned), c->st));
     launch_init_fluid<Real>(c->ph, d, b, c->reps[0].p.vel_law, c->nf_total, max_nf, c->stage_pos, c->stage_vel, mean,
                             fluid_of<Real>(c, 1 - c->cur), fluid_of<Real>(c, c->cur), fill, c->counts[c->cur], c->st);
     HIPCHK(c, hipStreamSynchronize(c->st));
@@ -1134,6 +1232,7 @@ extern "C" {
 
 BW_API int initialize_fluid(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (c->reps[0].p.fluid_init == BW_INIT_DEVICE)
         return c->fp64 ? init_fluid_device<double>(c) : init_fluid_device<float>(c);
@@ -1159,6 +1258,7 @@ BW_API int create_box(bw_ctx *c) {
 
 BW_API int tumble(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     for (int r = 0; r < c->n_rep; r++) {
         ReplicaHost &R = c->reps[r];
@@ -1175,6 +1275,7 @@ BW_API int tumble(bw_ctx *c) {
 
 BW_API int neighbour_list_mpcd(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     int rc = alloc_maps(c);
     if (rc) return rc;
     if (c->fp64)
@@ -1186,6 +1287,7 @@ BW_API int neighbour_list_mpcd(bw_ctx *c) {
 
 BW_API int neighbour_list_md(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     if (c->nc_total == 0) return BW_OK;
     Dev d = dev_for(c, c->cur);
     launch_md_candidates(c->ph, d, c->wgt, c->nwg, c->st);
@@ -1196,6 +1298,7 @@ BW_API int neighbour_list_md(bw_ctx *c) {
 #define COLLOID_ENTRY(name, flags)                                   \
     BW_API int name(bw_ctx *c) {                                     \
         if (!c) return BW_ERR_ARG;                                   \
+        SETTLE(c);                                                   \
         launch_colloid(c->ph, dev_for(c, c->cur), (flags), c->st);   \
         return BW_OK;                                                \
     }
@@ -1206,6 +1309,7 @@ COLLOID_ENTRY(bw_copy_old_force, PH_OLDF)
 
 BW_API int update_pos_md(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     if (c->nc_total == 0) return BW_OK;
     launch_colloid(c->ph, dev_for(c, c->cur), PH_POS, c->st);
     c->cb ^= 1;  // the new positions are in the other buffer
@@ -1214,6 +1318,7 @@ BW_API int update_pos_md(bw_ctx *c) {
 
 BW_API int rotation_mpcd(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     int rc = alloc_maps(c);
     if (rc) return rc;
     if ((rc = sync_injected(c))) return rc;
@@ -1234,6 +1339,7 @@ BW_API int rotation_mpcd(bw_ctx *c) {
 
 BW_API int run(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     Dev d = dev_for(c, c->cur);
     launch_colloid(c->ph, d, PH_KICK, c->st);
     if (c->nc_total == 0) return BW_OK;
@@ -1252,6 +1358,7 @@ BW_API int run(bw_ctx *c) {
 // needs the neigh_fl lists of neighbour_list_mpcd
 BW_API int updown_velocity(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     if (!c->maps_alloc) return fail(c, BW_ERR_STATE, "updown_velocity: call neighbour_list_mpcd first");
     int rc;
     const size_t NC = std::max(c->nc_total, 1);
@@ -1278,6 +1385,7 @@ BW_API int updown_velocity(bw_ctx *c) {
 BW_API int bw_get_updown(bw_ctx *c, int r, int *cnt, int *up_cnt, double *vel, double *up_vel) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
+    SETTLE(c);
     if (!c->ud_sums) return fail(c, BW_ERR_STATE, "bw_get_updown: updown_velocity not run");
     HIPCHK(c, hipStreamSynchronize(c->st));
     const size_t g0 = (size_t)R->first_colloid, n = (size_t)R->nc;
@@ -1290,6 +1398,7 @@ BW_API int bw_get_updown(bw_ctx *c, int r, int *cnt, int *up_cnt, double *vel, d
 
 BW_API int update_pos_mpcd(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     Dev d = dev_for(c, c->cur);
     if (c->fp64) launch_stream<double>(c->ph, d, c->fl[c->cur].f64, false, true, false, false, c->st);
     else launch_stream<float>(c->ph, d, c->fl[c->cur].f32, false, true, false, false, c->st);
@@ -1298,6 +1407,7 @@ BW_API int update_pos_mpcd(bw_ctx *c) {
 
 BW_API int fluid_colloid_collision(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     int rc = sync_injected(c);
     if (rc) return rc;
     if (c->nc_total == 0) return BW_OK;
@@ -1327,7 +1437,7 @@ BW_API int bw_startup(bw_ctx *c) {
 
 BW_API int bw_step(bw_ctx *c, int nsteps) {
     if (!c) return BW_ERR_ARG;
-    return c->fp64 ? do_steps<double>(c, nsteps) : do_steps<float>(c, nsteps);
+    return c->fp64 ? do_steps<double>(c, nsteps, nullptr) : do_steps<float>(c, nsteps, nullptr);
 }
 
 BW_API int bw_profile_steps(bw_ctx *c, int nsteps, double *ms, int *launches) {
@@ -1337,6 +1447,7 @@ BW_API int bw_profile_steps(bw_ctx *c, int nsteps, double *ms, int *launches) {
 
 BW_API int bw_time_steps(bw_ctx *c, int nsteps, double *ms) {
     if (!c || !ms) return BW_ERR_ARG;
+    SETTLE(c);
     hipEvent_t a, b;
     HIPCHK(c, hipEventCreate(&a));
     HIPCHK(c, hipEventCreate(&b));
@@ -1344,6 +1455,11 @@ BW_API int bw_time_steps(bw_ctx *c, int nsteps, double *ms) {
     int rc = bw_step(c, nsteps);
     HIPCHK(c, hipEventRecord(b, c->st));
     HIPCHK(c, hipEventSynchronize(b));
+    if (!rc && c->groups && *(volatile long long *)c->halt_step) {  // steps to take again belong to the time
+        rc = settle(c);
+        HIPCHK(c, hipEventRecord(b, c->st));
+        HIPCHK(c, hipEventSynchronize(b));
+    }
     float t = 0;
     hipEventElapsedTime(&t, a, b);
     *ms = t;
@@ -1356,6 +1472,7 @@ BW_API int bw_time_steps(bw_ctx *c, int nsteps, double *ms) {
 BW_API int bw_set_v0(bw_ctx *c, int r, const double *v0) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     for (int j = 0; j < R->nc; j++) R->v0[j] = v0 ? v0[j] : R->p.v0;
     if (R->nc)
@@ -1366,6 +1483,7 @@ BW_API int bw_set_v0(bw_ctx *c, int r, const double *v0) {
 BW_API int bw_upload_fluid(bw_ctx *c, int r, const double *pos, const double *vel) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !pos || !vel) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     return c->fp64 ? upload_fluid_impl<double>(c, r, pos, vel) : upload_fluid_impl<float>(c, r, pos, vel);
 }
@@ -1373,13 +1491,16 @@ BW_API int bw_upload_fluid(bw_ctx *c, int r, const double *pos, const double *ve
 BW_API int bw_download_fluid(bw_ctx *c, int r, double *pos, double *vel, int *cell) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
-    return c->fp64 ? download_fluid_impl<double>(c, r, pos, vel, cell) : download_fluid_impl<float>(c, r, pos, vel, cell);
+    return read_settled(c, [&]() {
+        return c->fp64 ? download_fluid_impl<double>(c, r, pos, vel, cell) : download_fluid_impl<float>(c, r, pos, vel, cell);
+    });
 }
 
 BW_API int bw_upload_colloid(bw_ctx *c, int r, const double *pos, const double *vel, const double *omega,
                              const double *f, const double *old_f, const double *ra) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     size_t o = 3 * (size_t)R->first_colloid, n = sizeof(double) * 3 * R->nc;
     if (!R->nc) return BW_OK;
@@ -1400,19 +1521,23 @@ BW_API int bw_download_colloid(bw_ctx *c, int r, double *pos, double *vel, doubl
                                double *ra) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
-    const size_t o = 3 * (size_t)R->first_colloid, n = sizeof(double) * 3 * R->nc;
-    const StageSeg seg[] = {{pos, c->cposb[c->cb] + o, n}, {vel, c->dv.cvel + o, n},   {omega, c->dv.comega + o, n},
-                            {f, c->dv.cf + o, n},          {old_f, c->dv.coldf + o, n}, {ra, c->dv.cra + o, n}};
-    HIPCHK(c, c->staging.download(seg, 6, c->st));
-    return BW_OK;
+    return read_settled(c, [&]() -> int {
+        const size_t o = 3 * (size_t)R->first_colloid, n = sizeof(double) * 3 * R->nc;
+        const StageSeg seg[] = {{pos, c->cposb[c->cb] + o, n}, {vel, c->dv.cvel + o, n},   {omega, c->dv.comega + o, n},
+                                {f, c->dv.cf + o, n},          {old_f, c->dv.coldf + o, n}, {ra, c->dv.cra + o, n}};
+        HIPCHK(c, c->staging.download(seg, 6, c->st));
+        return BW_OK;
+    });
 }
 
 BW_API int bw_download_displacement(bw_ctx *c, int r, double *disp) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !disp) return BW_ERR_ARG;
     const StageSeg seg = {disp, c->dv.cdisp + 3 * (size_t)R->first_colloid, sizeof(double) * 3 * R->nc};
-    HIPCHK(c, c->staging.download(&seg, 1, c->st));
-    return BW_OK;
+    return read_settled(c, [&]() -> int {
+        HIPCHK(c, c->staging.download(&seg, 1, c->st));
+        return BW_OK;
+    });
 }
 
 BW_API int bw_rng_state(bw_ctx *c, int r, int *out36) {
@@ -1426,6 +1551,7 @@ BW_API int bw_rng_state(bw_ctx *c, int r, int *out36) {
 BW_API int bw_inject_rotation(bw_ctx *c, int r, const double *shift3, const double *axes) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || c->ph.draws != BW_DRAWS_INJECTED) return BW_ERR_ARG;
+    SETTLE(c);
     for (int k = 0; k < 3; k++) R->inj_shift[k] = shift3 ? shift3[k] : NAN;
     if (axes) R->inj_axes.assign(axes, axes + 2 * (size_t)R->cells);
     else R->inj_axes.assign(2 * (size_t)R->cells, NAN);
@@ -1437,6 +1563,7 @@ BW_API int bw_inject_reflections(bw_ctx *c, int r, int l, int n, const int *coll
                                  const double *vals6) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || c->ph.draws != BW_DRAWS_INJECTED || l < 0 || l >= c->ph.n_sub || n < 0) return BW_ERR_ARG;
+    SETTLE(c);
     R->inj_c[l].assign(colloid, colloid + n);
     R->inj_p[l].assign(particle, particle + n);
     R->inj_v[l].assign(vals6, vals6 + 6 * (size_t)n);
@@ -1448,6 +1575,7 @@ BW_API int bw_inject_reflections(bw_ctx *c, int r, int l, int n, const int *coll
 
 BW_API int bw_clear_injected(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     for (auto &R : c->reps) {
         for (int l = 0; l < c->ph.n_sub; l++) {
             R.inj_c[l].clear(); R.inj_p[l].clear(); R.inj_v[l].clear();
@@ -1463,6 +1591,7 @@ BW_API int bw_clear_injected(bw_ctx *c) {
 BW_API int bw_get_cell_lists(bw_ctx *c, int r, int *counts, int *list) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !c->maps_alloc) return BW_ERR_STATE;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (counts) HIPCHK(c, hipMemcpy(counts, c->dv.map_count + R->first_cell, sizeof(int) * R->cells, hipMemcpyDeviceToHost));
     if (list) HIPCHK(c, hipMemcpy(list, c->dv.map_list + R->first_fluid, sizeof(int) * R->nf, hipMemcpyDeviceToHost));
@@ -1472,6 +1601,7 @@ BW_API int bw_get_cell_lists(bw_ctx *c, int r, int *counts, int *list) {
 BW_API int bw_get_neigh_fl(bw_ctx *c, int r, int *counts, int *list, int cap) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !c->maps_alloc) return BW_ERR_STATE;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (!R->nc) return 0;
     std::vector<int> cnt(R->nc);
@@ -1493,6 +1623,7 @@ BW_API int bw_get_neigh_fl(bw_ctx *c, int r, int *counts, int *list, int cap) {
 BW_API int bw_get_md_list(bw_ctx *c, int r, int *counts, int *list, int cap) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (!R->nc) return 0;
     std::vector<int> cnt(R->nc), full((size_t)R->nc * MD_CAP);
@@ -1521,6 +1652,7 @@ BW_API int bw_get_md_list(bw_ctx *c, int r, int *counts, int *list, int cap) {
 BW_API int bw_get_shifted_cells(bw_ctx *c, int r, int *cells) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !c->maps_alloc || !cells) return BW_ERR_STATE;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     HIPCHK(c, hipMemcpy(cells, c->dv.shifted_cell + R->first_fluid, sizeof(int) * R->nf, hipMemcpyDeviceToHost));
     return BW_OK;
@@ -1529,6 +1661,7 @@ BW_API int bw_get_shifted_cells(bw_ctx *c, int r, int *cells) {
 BW_API int bw_get_run_counts(bw_ctx *c, int r, int *cnt) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !cnt) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (R->nc) HIPCHK(c, hipMemcpy(cnt, c->dv.ccnt + R->first_colloid, sizeof(int) * R->nc, hipMemcpyDeviceToHost));
     return BW_OK;
@@ -1556,14 +1689,16 @@ int fluid_sums(bw_ctx *c, const ReplicaHost &R, double *s, const StageSeg *more,
 BW_API int bw_audit(bw_ctx *c, int r, double *out) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !out) return BW_ERR_ARG;
-    if (R->nc) launch_potential(c->ph, dev_for(c, c->cur), r, c->st);
     const size_t n3 = 3 * (size_t)R->nc, o = 3 * (size_t)R->first_colloid;
     std::vector<double> v(n3), w(n3);
     double pot = 0, s[5];
     const StageSeg seg[] = {{v.data(), c->dv.cvel + o, sizeof(double) * n3},
                             {w.data(), c->dv.comega + o, sizeof(double) * n3},
                             {&pot, c->dv.cpot + r, R->nc ? sizeof(double) : 0}};
-    const int rc = fluid_sums(c, *R, s, seg, 3);
+    const int rc = read_settled(c, [&]() {
+        if (R->nc) launch_potential(c->ph, dev_for(c, c->cur), r, c->st);
+        return fluid_sums(c, *R, s, seg, 3);
+    });
     if (rc) return rc;
     double kec = 0, ang = 0, pc[3] = {0, 0, 0}, absm = 0;
     for (int i = 0; i < R->nc; i++) {
@@ -1619,6 +1754,7 @@ BW_API int bw_host_initialize(const bw_params *p, double *pos_fl, double *vel_fl
 
 BW_API int bw_observables_reset(bw_ctx *c) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     size_t NC = std::max(c->nc_total, 1);
     HIPCHK(c, hipMemsetAsync(c->dv.cdisp, 0, sizeof(double) * 3 * NC, c->st));
@@ -1643,7 +1779,7 @@ BW_API int bw_observables(bw_ctx *c, int r, double *out) {
                             {v.data(), c->dv.cvel + o, sizeof(double) * n3},
                             {w.data(), c->dv.comega + o, sizeof(double) * n3}};
     double s[5];
-    const int rc = fluid_sums(c, *R, s, seg, 4);
+    const int rc = read_settled(c, [&]() { return fluid_sums(c, *R, s, seg, 4); });
     if (rc) return rc;
     const double m = R->p.mass_fl, N = (double)R->nf;
     const double ke = 0.5 * s[3] * m, px = s[0] * m, py = s[1] * m, pz = s[2] * m;
@@ -1674,6 +1810,7 @@ BW_API int bw_observables(bw_ctx *c, int r, double *out) {
 
 BW_API int bw_set_moments(bw_ctx *c, int on) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     if (on && !c->moments_ok) return fail(c, BW_ERR_ARG, "coarse moments need even box and tile edges");
     if (!on && c->ph.surrogate) return fail(c, BW_ERR_STATE, "the attached surrogate needs the moments");
     HIPCHK(c, hipStreamSynchronize(c->st));
@@ -1687,6 +1824,7 @@ BW_API int bw_set_moments(bw_ctx *c, int on) {
 BW_API int bw_surrogate_attach(bw_ctx *c, bw_mlp *m, const float *lo, const float *hi, const float *t_lo,
                                const float *t_hi) {
     if (!c) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     destroy_graphs(c);
     if (!m) {
@@ -1735,6 +1873,7 @@ BW_API int bw_surrogate_attach(bw_ctx *c, bw_mlp *m, const float *lo, const floa
 BW_API int bw_get_surrogate_data(bw_ctx *c, int r, float *feat, double *imp, int *mode) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (!R->nc) return BW_OK;
     size_t g0 = (size_t)R->first_colloid;
@@ -1748,6 +1887,7 @@ BW_API int bw_get_surrogate_data(bw_ctx *c, int r, float *feat, double *imp, int
 BW_API int bw_get_surrogate_shells(bw_ctx *c, int r, int *count, double *sums) {
     ReplicaHost *R = rep_of(c, r);
     if (!R) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (!R->nc) return BW_OK;
     size_t g0 = (size_t)R->first_colloid;
@@ -1761,9 +1901,17 @@ BW_API int bw_get_surrogate_shells(bw_ctx *c, int r, int *count, double *sums) {
     return BW_OK;
 }
 
+BW_API int bw_step_paths(bw_ctx *c, long long *out3) {
+    if (!c || !out3) return BW_ERR_ARG;
+    SETTLE(c);
+    std::copy(c->path_steps, c->path_steps + 3, out3);
+    return BW_OK;
+}
+
 BW_API int bw_near_particles(bw_ctx *c, int r, long long *n_near) {
     ReplicaHost *R = rep_of(c, r);
     if (!R || !n_near) return BW_ERR_ARG;
+    SETTLE(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
     std::vector<int> cnt(R->n_tiles);
     HIPCHK(c, hipMemcpy(cnt.data(), c->dv.near_cnt + R->first_tile, sizeof(int) * R->n_tiles, hipMemcpyDeviceToHost));

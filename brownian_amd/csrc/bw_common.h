@@ -48,6 +48,7 @@ constexpr int GROUP_MAX = 24;       // colloids of a group that a workgroup of i
 // us, with 640 already 554 against 485)
 constexpr int GROUP_WIDE = 512;
 constexpr int GROUP_LDS_COLLOIDS = 3072;  // colloids that k_group_lists holds in LDS
+constexpr int SAVE_WORDS = 47;  // state of a colloid that a step by groups changes in place
 constexpr int OVL_CAP = 65536;      // hot particles beyond a full bucket, all colloids
 constexpr long long MEAN_CHUNK = 65536;  // particles per workgroup of the start-up's mean
 // workgroups per replica of the start-up's mean for replicas of up to max_nf particles
@@ -172,12 +173,12 @@ struct Dev {
     int *hot_cnt, *hot_ent;  // per colloid: slots of the particles that may reach it in the step
     int hot_cap;
     int *ovl_cnt, *ovl_g, *ovl_slot;  // entries beyond a full bucket
-    int *redo;           // per colloid: its group is left to k_groups_redo
-    int *redo_list;      // per replica (at its first colloid): those colloids
-    int *redo_cnt;       // per replica
-    int *redo_mark;      // the last step that redid any, the number of such steps, the most colloids in one
-    int *redo_stat;      // the last two in host memory
-    unsigned *status;
+    // a step by groups that could not be finished so: nonzero until the host
+    // has taken it again; the kernels of the steps after it return at once
+    int *halt;
+    long long *halt_step;  // its number, in host memory
+    long long *save;       // SAVE_WORDS words per colloid: its state at the step's start
+    unsigned *status;      // [0] flags, [1] those of the present step by groups
     long long *step;     // MPCD step counter (device generator key)
     double *shift;       // [n_rep*3] shift of the current step
     // injected draws

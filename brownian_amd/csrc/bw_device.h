@@ -460,6 +460,41 @@ __device__ inline void group_join(const Dev &d, int a, int b) {
         if (atomicCAS(&d.uf[a], a, b) == a) return;  // a was a root: now below b < a
     }
 }
+// A step by groups that cannot be finished so (a group beyond the lists) is
+// stopped: its kernels and those of the steps already launched behind it return
+// at once, until the host has put the colloids' state back (k_restore) and
+// taken the step kernel by kernel.  The fluid buffer that the step started from
+// is whole until the next one.
+__device__ __forceinline__ bool stopped(const Phys &ph, const Dev &d) { return ph.groups && ld_const(d.halt) != 0; }
+__device__ inline void stop_step(const Dev &d) {  // any number of threads
+    *(volatile int *)d.halt = 1;
+    *(volatile long long *)d.halt_step = *d.step;
+}
+// word i of the state of colloid g that a step by groups changes in place
+__device__ inline long long *colloid_word(const Dev &d, int g, int i) {
+    const int k = i % 3;
+    switch (i / 3) {
+        case 0: return (long long *)d.cvel + 3 * g + k;
+        case 1: return (long long *)d.comega + 3 * g + k;
+        case 2: return (long long *)d.cra + 3 * g + k;
+        case 3: return (long long *)d.cf + 3 * g + k;
+        case 4: return (long long *)d.coldf + 3 * g + k;
+        case 5: return (long long *)d.cdisp + 3 * g + k;
+        case 6: return (long long *)d.cpos_run + 3 * g + k;
+        case 7:
+        case 8: return (long long *)d.cimp + 6 * g + i - 21;
+        default: return (long long *)d.sacc + SUR_ACC * g + i - 27;
+    }
+}
+__device__ inline int *colloid_int(const Dev &d, int g, int i) {
+    return i < 3 ? d.ccell_run + 3 * g + i : i == 3 ? d.ccnt + g : d.sshell + g;
+}
+constexpr int SAVE_LONG = 27 + SUR_ACC;
+static_assert(SAVE_WORDS == SAVE_LONG + 5, "colloid_word, colloid_int");
+__device__ inline void save_colloid(const Dev &d, int g, int i, int n) {  // thread i of n
+    long long *w = d.save + (size_t)SAVE_WORDS * g;
+    for (; i < SAVE_WORDS; i += n) w[i] = i < SAVE_LONG ? *colloid_word(d, g, i) : *colloid_int(d, g, i - SAVE_LONG);
+}
 // Colloids that can touch a particle of a tile during one MPCD step: a
 // particle stays within TILE_REACH cells of its tile box, the collision and
 // run() stencils reach 3 cells and a colloid's cell moves by at most one cell

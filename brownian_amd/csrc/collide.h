@@ -1,7 +1,6 @@
 // The per-substep work of one colloid's collisions, of a replica's serial
-// replay and of a colloid's update, as device functions: the per-substep
-// kernels call them from one launch each, k_groups_redo in turn from one
-// workgroup.
+// replay and of a colloid's update, as device functions of the per-substep
+// kernels; reflect_event and transfer are k_groups' too.
 #pragma once
 #include "bw_device.h"
 
@@ -248,7 +247,7 @@ struct SerialLds {
 };
 template <class Real>
 __device__ __forceinline__ void serial_replay(const Phys &ph, const Dev &d, const Fluid<Real> &f, int substep, int r,
-                                              bool check, SerialLds &sh) {
+                                              SerialLds &sh) {
     const bool fp32 = sizeof(Real) == 4;
     const Rep R = d.rep[r];
     const int L = R.L;
@@ -348,7 +347,7 @@ __device__ __forceinline__ void serial_replay(const Phys &ph, const Dev &d, cons
             __syncthreads();
         }
     }
-    if (check && ph.draws == BW_DRAWS_INJECTED) {
+    if (ph.draws == BW_DRAWS_INJECTED) {
         // every GPU event found its (colloid, particle) tuple; equal totals
         // then mean equal sets
         int my_inj = 0;
@@ -366,7 +365,7 @@ __device__ __forceinline__ void serial_replay(const Phys &ph, const Dev &d, cons
         d.chain_cnt[r] = 0;
         d.cont_cnt[r] = 0;
         d.ovf_cnt[r] = 0;
-        d.ev_total[r] = check ? 0 : d.ev_total[r] + sh.serial_events;
+        d.ev_total[r] = 0;
     }
 }
 

@@ -8,9 +8,11 @@
 // k_groups runs all n_sub substeps of a group in one wave or workgroup
 // (streaming, stochastic reflection in the reference's event order, serial
 // replay, WCA forces, Verlet, activity), with the colloids in LDS, in place of
-// four launches per substep over all of them.  Those are bound by latency: 28 us
-// a substep with 8 colloids (20^3), 35 with 300 (64^3), 54 with 2400 (128^3),
-// of which the kernels' first loads are most.  20 substeps by groups, with the
+// four launches per substep over all of them.  A step that has a group of more
+// colloids or events than these lists hold is stopped (stop_step) and taken
+// again kernel by kernel.  The launches are bound by latency: 28 us a substep
+// with 8 colloids (20^3), 35 with 300 (64^3), 54 with 2400 (128^3), of which
+// the kernels' first loads are most.  20 substeps by groups, with the
 // classification and the lists, take 0.19, 0.25 and 0.39 ms in place of 0.56,
 // 0.69 and 1.06 (FP32; FP64 at 20^3).
 #include "bw_device.h"
@@ -302,8 +304,7 @@ __device__ __forceinline__ bool reflect_quad(const Phys &ph, const Rep &R, const
 // keeps the selected particles at about one per lane (6 per colloid and substep
 // at 10 particles per cell and 20 substeps).
 //
-// False: beyond the LDS lists' capacities (nothing is stored then that
-// k_groups_redo does not store again; the global state is written at the end).
+// False: beyond the LDS lists' capacities.
 template <class Real, int NW>
 __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const Fluid<Real> &f, HotPart<Real> *h, int final,
                                            int n_col, int r, GroupLds<Real, NW> &s) {
@@ -362,16 +363,13 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
         }
     }
     if (tid < 14) s.cnt[0][tid] = 0;
-    bool full = false;  // a bucket overflowed
     int n_hot = 0;
     for (int c = 0; c < C; c++) {
         const int n = d.hot_cnt[s.g[c]];
         if (tid == 0) s.hot[c] = n_hot;
         n_hot += n;
-        full = full || n > d.hot_cap;
     }
     if (tid == 0) s.hot[C] = n_hot;
-    if (full) return false;
     h += d.grp_hot[s.g[0]];  // the group's working copies
     int *slots = d.grp_slot + d.grp_hot[s.g[0]];
     sync();
@@ -835,18 +833,18 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
 }
 
 // The groups' lists, by one workgroup: every colloid's root, the sizes, then
-// per group of up to GROUP_MAX colloids its members (in any order) and its
-// place among the large groups or the small ones.  Larger groups go to
-// k_groups_redo.
+// per group its members (in any order) and its place among the large groups or
+// the small ones.  A group of more than GROUP_MAX colloids or with a full bucket
+// ends the step here.
 __global__ __launch_bounds__(1024) void k_group_lists(Phys ph, Dev d) {
     // roots, sizes, numbers of particles, places: in LDS while they fit
     __shared__ int s_arr[4][GROUP_LDS_COLLOIDS];
-    __shared__ int s_mem, s_hot, s_big, s_small;
+    __shared__ int s_mem, s_hot, s_big, s_small, s_over;
     const int nc = ph.n_colloid_total;
     const bool lds = nc <= GROUP_LDS_COLLOIDS;
     int *root = lds ? s_arr[0] : d.grp_root, *size = lds ? s_arr[1] : d.grp_root + nc,
         *off = lds ? s_arr[2] : d.grp_root + 2 * (size_t)nc, *hot = lds ? s_arr[3] : d.grp_root + 3 * (size_t)nc;
-    if (threadIdx.x == 0) { s_mem = 0; s_hot = 0; s_big = 0; s_small = 0; }
+    if (threadIdx.x == 0) { s_mem = 0; s_hot = 0; s_big = 0; s_small = 0; s_over = 0; }
     for (int g = threadIdx.x; g < nc; g += 1024) {
         size[g] = 0;
         hot[g] = 0;
@@ -863,13 +861,14 @@ __global__ __launch_bounds__(1024) void k_group_lists(Phys ph, Dev d) {
         const int p = d.uf_linked[g] ? group_find(d, g) : g;
         root[g] = p;
         atomicAdd(&size[p], 1);
-        atomicAdd(&hot[p], min(n, d.hot_cap));
+        atomicAdd(&hot[p], n);
+        if (n > d.hot_cap) s_over = 1;
     }
     sync();
     for (int g = threadIdx.x; g < nc; g += 1024) {
         if (root[g] != g) continue;
         const int C = size[g];
-        if (C > GROUP_MAX) continue;
+        if (C > GROUP_MAX) s_over = 1;
         const int o = atomicAdd(&s_mem, C);
         d.grp_hot[g] = atomicAdd(&s_hot, hot[g]);
         if (C > GROUP_SMALL || nc <= GROUP_WIDE) d.grp_big[atomicAdd(&s_big, 1)] = make_int2(o, C);
@@ -877,15 +876,12 @@ __global__ __launch_bounds__(1024) void k_group_lists(Phys ph, Dev d) {
         off[g] = o;
     }
     sync();
-    for (int g = threadIdx.x; g < nc; g += 1024) {
-        const int p = root[g];
-        if (size[p] <= GROUP_MAX) {
-            d.grp_mem[atomicAdd(&off[p], 1)] = g;
-        } else {
-            d.redo[g] = 1;
-            atomicAdd(&d.redo_cnt[d.crep[g]], 1);
-        }
+    if (stopped(ph, d)) return;
+    if (s_over) {
+        if (threadIdx.x == 0) stop_step(d);
+        return;
     }
+    for (int g = threadIdx.x; g < nc; g += 1024) d.grp_mem[atomicAdd(&off[root[g]], 1)] = g;
     if (threadIdx.x == 0) {
         d.grp_cnt[0] = s_big;
         d.grp_cnt[1] = s_small;
@@ -909,6 +905,7 @@ __global__ __launch_bounds__(256, WIDE || sizeof(Real) == 8 ? 2 : 3) void k_grou
         GroupLds<Real, 1> small[WIDE ? 1 : 4];
     } s;
     const int n_big = ld_const(d.grp_cnt), n_small = WIDE ? 0 : ld_const(d.grp_cnt + 1);
+    if (stopped(ph, d)) return;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // members in ascending order into g[0..C)
     auto members = [&](int2 grp, int *g) {
@@ -917,16 +914,12 @@ __global__ __launch_bounds__(256, WIDE || sizeof(Real) == 8 ? 2 : 3) void k_grou
         for (int j = 0; j < grp.y; j++) rank += lane_value(v, j) < v ? 1 : 0;
         if (lane < grp.y) g[rank] = v;
     };
-    auto left = [&](const int *g, int C, int r, int i0, int n) {  // to k_groups_redo
-        for (int c = i0; c < C; c += n) d.redo[g[c]] = 1;
-        if (i0 == 0) atomicAdd(&d.redo_cnt[r], C);
-    };
     if ((int)blockIdx.x < n_big) {
         const int2 grp = ld_const(d.grp_big + blockIdx.x);
         if (w == 0) members(grp, s.big.g);
         __syncthreads();
         const int r = __builtin_amdgcn_readfirstlane(d.crep[s.big.g[0]]);
-        if (!group_step<Real, 4>(ph, d, f, h, final, grp.y, r, s.big)) left(s.big.g, grp.y, r, threadIdx.x, 256);
+        if (!group_step<Real, 4>(ph, d, f, h, final, grp.y, r, s.big)) stop_step(d);
     } else if constexpr (!WIDE) {
         const int i = ((int)blockIdx.x - n_big) * 4 + w;
         if (i >= n_small) return;
@@ -934,172 +927,35 @@ __global__ __launch_bounds__(256, WIDE || sizeof(Real) == 8 ? 2 : 3) void k_grou
         members(grp, s.small[w].g);
         wave_sync();
         const int r = __builtin_amdgcn_readfirstlane(d.crep[s.small[w].g[0]]);
-        if (!group_step<Real, 1>(ph, d, f, h, final, grp.y, r, s.small[w])) left(s.small[w].g, grp.y, r, lane, 64);
+        if (!group_step<Real, 1>(ph, d, f, h, final, grp.y, r, s.small[w])) stop_step(d);
     }
 }
 
-// The groups that k_groups left (more colloids, events or serially replayed
-// particles than its lists hold, a full bucket): the colloids of all of them, per replica, as
-// one group without bounds, by one workgroup, with the per-substep kernels'
-// own functions and lists in global memory.  Rare; otherwise it returns at
-// once.  With injected draws it also checks the step's totals.
-template <class Real>
-__global__ __launch_bounds__(COLLIDE_THREADS) void k_groups_redo(Phys ph, Dev d, Fluid<Real> f, int final) {
-    constexpr int NW = COLLIDE_THREADS / 64;
-    __shared__ union {
-        CollideLds c[NW];
-        SerialLds s;
-        UpdateLds u[NW];
-    } sh;
-    __shared__ int s_wt[16];
+// With injected draws, after k_groups: every event found its tuple; equal
+// totals over the step then mean equal sets
+__global__ __launch_bounds__(256) void k_check_draws(Phys ph, Dev d) {
     __shared__ int s_tot;
-    const int r = blockIdx.x, tid = threadIdx.x;
-    const int n = ld_const(d.redo_cnt + r);
-    if (n == 0 && ph.draws != BW_DRAWS_INJECTED) return;
-    const Rep R = d.rep[r];
-    const int L = R.L, g_end = R.first_colloid + R.nc;
-    const double Ld = (double)L;
-    int *list = d.redo_list + R.first_colloid;
-    if (n > 0) {
-        int cnt = 0;
-        for (int base = R.first_colloid; base < g_end; base += COLLIDE_THREADS) {
-            const int g = base + tid;
-            const bool p = g < g_end && d.redo[g];
-            int tot;
-            const int idx = block_compact(p, s_wt, tot);
-            if (p) list[cnt + idx] = g;
-            cnt += tot;
-        }
-        __threadfence();
-        __syncthreads();
-        Dev dd = d;
-        const int n_ovl = min(*d.ovl_cnt, OVL_CAP);
-        bool drift = false, ch_over = false, escaped = false;
-        auto sync = [&]() {  // global stores of one phase before the loads of the next
-            __threadfence();
-            __syncthreads();
-        };
-        for (int l = 0; l < ph.n_sub; l++) {
-            const bool last = l == ph.n_sub - 1;
-            auto stream = [&](int slot) {
-                const int c0 = f.cell[slot];
-                int phantom = c0 & PHANTOM;
-                int ix, iy, iz;
-                unpack_cell(c0, ix, iy, iz);
-                Real ox = f.ox[slot], oy = f.oy[slot], oz = f.oz[slot];
-                const Real vx = f.vx[slot], vy = f.vy[slot], vz = f.vz[slot];
-                const double vn = sqrt(((double)vx * vx + (double)vy * vy) + (double)vz * vz);
-                if (vn * ph.ndt > ph.group_reach &&
-                    reaches_other(ph, d, R, (double)ix + (double)ox, (double)iy + (double)oy, (double)iz + (double)oz, vn, l - 1,
-                                  [&](int g) { return d.redo[g] != 0; }))
-                    escaped = true;
-                fly_flat(1, (Real)ph.dt, L, vx, vy, vz, ix, iy, iz, ox, oy, oz);
-                if (outside_tile_reach(R, ph.cap, slot, ix, iy, iz)) drift = true;
-                const double x = (double)ix + (double)ox, y = (double)iy + (double)oy, z = (double)iz + (double)oz;
-                int n_in = 0, gin = -1;
-                bool inside = false;
-                for (int m = 0; m < cnt; m++) {
-                    const int g = list[m];
-                    const int cx = dd.ccell[3 * g], cy = dd.ccell[3 * g + 1], cz = dd.ccell[3 * g + 2];
-                    const int ax = pdiff(ix, cx, L), ay = pdiff(iy, cy, L), az = pdiff(iz, cz, L);
-                    if (ax < -3 || ax > 3 || ay < -3 || ay > 3 || az < -3 || az > 3) continue;
-                    if (ph.surrogate && d.cmode[g]) continue;
-                    const double rx = img1(dd.cpos[3 * g] - x, Ld), ry = img1(dd.cpos[3 * g + 1] - y, Ld),
-                                 rz = img1(dd.cpos[3 * g + 2] - z, Ld);
-                    if ((rx * rx + ry * ry) + rz * rz <= ph.lim_coll) {
-                        inside = true;
-                        if (in_stencil(ix, iy, iz, cx, cy, cz, L)) {
-                            n_in++;
-                            gin = g;
-                        }
-                    }
-                }
-                if (phantom) {
-                    if (!inside) phantom = 0;
-                    n_in = 0;
-                }
-                f.cell[slot] = pack_cell(ix, iy, iz) | phantom;
-                f.ox[slot] = ox; f.oy[slot] = oy; f.oz[slot] = oz;
-                if (n_in > 0) {
-                    const int e = n_in == 1 ? atomicAdd(&d.ev_cnt[gin], 1) : EV_CAP;
-                    if (e < EV_CAP) {
-                        d.ev_slot[gin * EV_CAP + e] = slot;
-                    } else {
-                        const int e2 = atomicAdd(&d.chain_cnt[r], 1);
-                        if (e2 < CHAIN_CAP) d.chain_slot[r * CHAIN_CAP + e2] = slot;
-                        else ch_over = true;
-                    }
-                }
-            };
-            for (int m = 0; m < cnt; m++) {
-                const int g = list[m], nb = min(d.hot_cnt[g], d.hot_cap);
-                for (int e = tid; e < nb; e += COLLIDE_THREADS)
-                    stream(d.hot_ent[(size_t)g * d.hot_cap + e]);
-            }
-            for (int e = tid; e < n_ovl; e += COLLIDE_THREADS) {
-                const int g = d.ovl_g[e];
-                if (g >= R.first_colloid && g < g_end && d.redo[g]) stream(d.ovl_slot[e]);
-            }
-            sync();
-            for (int m = tid >> 6; m < cnt; m += NW) collide_wave<Real>(ph, dd, f, l, r, list[m], sh.c[tid >> 6]);
-            sync();
-            serial_replay<Real>(ph, dd, f, l, r, false, sh.s);
-            sync();
-            unsigned flags = PH_APPLY | PH_ACTIVITY | PH_FORCE | PH_VELOCITY;
-            if (!last) flags |= PH_OLDF | PH_POS | PH_MARGIN;
-            else if (!final) flags |= PH_KICK | PH_OLDF | PH_POS;
-            for (int m = tid >> 6; m < cnt; m += NW) colloid_update_wave(ph, dd, flags, r, list[m], sh.u[tid >> 6]);
-            sync();
-            if (flags & PH_POS) {
-                double *p = dd.cpos;
-                dd.cpos = dd.cpos_nxt;
-                dd.cpos_nxt = p;
-                int *q = dd.ccell;
-                dd.ccell = dd.ccell_nxt;
-                dd.ccell_nxt = q;
-            }
-        }
-        if (dd.cpos == d.cpos)  // an even number of position updates
-            for (int i = tid; i < 3 * cnt; i += COLLIDE_THREADS) {
-                const int j = 3 * list[i / 3] + i % 3;
-                d.cpos_nxt[j] = d.cpos[j];
-                d.ccell_nxt[j] = d.ccell[j];
-            }
-        if (drift) atomicOr(d.status, BW_FLAG_DRIFT);
-        if (ch_over) atomicOr(d.status, BW_FLAG_CHAIN_OVERFLOW);
-        if (escaped) atomicOr(d.status, BW_FLAG_MARGIN);
-        sync();
-        for (int m = tid; m < cnt; m += COLLIDE_THREADS) d.redo[list[m]] = 0;
-        if (tid == 0) {
-            d.redo_cnt[r] = 0;
-            // for the host's choice of the next steps' path: steps that redid
-            // any, and the largest number of colloids
-            const int step = (int)*d.step;
-            if (atomicMax(d.redo_mark, step) < step) ((volatile int *)d.redo_stat)[0] = atomicAdd(d.redo_mark + 1, 1) + 1;
-            if (n > atomicMax(d.redo_mark + 2, n)) ((volatile int *)d.redo_stat)[1] = n;
-        }
+    if (stopped(ph, d)) return;
+    const Rep R = d.rep[blockIdx.x];
+    if (threadIdx.x == 0) s_tot = 0;
+    __syncthreads();
+    int mine = 0;
+    for (int i = threadIdx.x; i < ph.n_sub * R.nc; i += 256) {
+        const int b = (i / R.nc) * ph.n_colloid_total + R.first_colloid + i % R.nc;
+        mine += d.inj_off[b + 1] - d.inj_off[b];
     }
-    if (ph.draws == BW_DRAWS_INJECTED) {
-        // every event found its tuple; equal totals then mean equal sets
-        if (tid == 0) s_tot = 0;
-        __syncthreads();
-        int mine = 0;
-        for (int i = tid; i < ph.n_sub * R.nc; i += COLLIDE_THREADS) {
-            const int b = (i / R.nc) * ph.n_colloid_total + R.first_colloid + i % R.nc;
-            mine += d.inj_off[b + 1] - d.inj_off[b];
-        }
-        atomicAdd(&s_tot, mine);
-        __syncthreads();
-        if (tid == 0) {
-            if (s_tot != d.ev_total[r]) atomicOr(d.status, BW_FLAG_DRAW_MISMATCH);
-            d.ev_total[r] = 0;
-        }
+    atomicAdd(&s_tot, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_tot != d.ev_total[blockIdx.x]) atomicOr(d.status, BW_FLAG_DRAW_MISMATCH);
+        d.ev_total[blockIdx.x] = 0;
     }
 }
 
 // The pair list at the colloids' present positions (cpp/neighbour_list.cpp:27-39),
 // a wave per colloid: what the per-substep path leaves after its last substep
 __global__ __launch_bounds__(256) void k_pair_lists(Phys ph, Dev d, const int2 *wgt) {
+    if (stopped(ph, d)) return;
     const int lane = threadIdx.x & 63;
     const int2 wt = wgt[blockIdx.x];
     const int r = wt.x, g = wt.y + (threadIdx.x >> 6);
@@ -1134,7 +990,7 @@ void launch_groups(const Phys &ph, const Dev &d, const Fluid<Real> &f, HotPart<R
     const GroupArgs<Real> a{ph, d, f, h, (int)final};
     if (ph.n_colloid_total <= GROUP_WIDE) hipLaunchKernelGGL((k_groups<Real, true>), dim3(ph.n_colloid_total), dim3(256), 0, st, a);
     else hipLaunchKernelGGL((k_groups<Real, false>), dim3(ph.n_colloid_total / 2 + 1), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(k_groups_redo<Real>, dim3(ph.n_rep), dim3(COLLIDE_THREADS), 0, st, ph, d, f, (int)final);
+    if (ph.draws == BW_DRAWS_INJECTED) hipLaunchKernelGGL(k_check_draws, dim3(ph.n_rep), dim3(256), 0, st, ph, d);
 }
 template void launch_groups<float>(const Phys &, const Dev &, const Fluid<float> &, HotPart<float> *, bool, hipStream_t);
 template void launch_groups<double>(const Phys &, const Dev &, const Fluid<double> &, HotPart<double> *, bool,

@@ -12,9 +12,9 @@
 // then the substeps, either by colloid groups (groups.hip, the usual way):
 //   k_classify         run() kick, first streaming, particles that may reach
 //                      a colloid into its bucket (the others fly the step)   (near chunks)
-//   k_group_lists, k_groups, k_groups_redo
+//   k_group_lists, k_groups
 // or kernel by kernel (BW_STREAM_PER_SUBSTEP, boxes whose colloids form large
-// groups):
+// groups, steps that k_groups could not finish):
 //   n_sub x { k_stream / k_stream_near  streaming, detection
 //             k_collide         1 wave / colloid: pair list, reflections
 //             k_serial          1 WG / replica: serial replays
@@ -43,7 +43,7 @@ __global__ void k_step_begin(Phys ph, Dev d, int clear_lists) {
                 d.hot_cnt[g] = 0;
             }
     }
-    if (blockIdx.x != 0) return;
+    if (blockIdx.x != 0 || stopped(ph, d)) return;
     long long s = *d.step + 1;
     for (int r = threadIdx.x; r < ph.n_rep; r += blockDim.x) {
         double u[3];
@@ -62,12 +62,37 @@ __global__ void k_step_begin(Phys ph, Dev d, int clear_lists) {
     if (threadIdx.x == 0) {
         *d.step = s;
         *d.chunk_cnt = 0;
-        if (ph.groups) *d.ovl_cnt = 0;
+        if (ph.groups) {
+            *d.ovl_cnt = 0;
+            // the last step by groups was not stopped: its flags count
+            if (d.status[1]) atomicOr(d.status, d.status[1]);
+            d.status[1] = 0;
+        }
+    }
+}
+
+// A stopped step's start again: the colloids, a workgroup each (their positions
+// and the fluid are in the buffers that the step read), the step number, and
+// what the step left behind.  The step taken again counts up to the same number.
+__global__ __launch_bounds__(64) void k_restore(Phys ph, Dev d) {
+    const int g = blockIdx.x;
+    const long long *w = d.save + (size_t)SAVE_WORDS * g;
+    for (int i = threadIdx.x; i < SAVE_WORDS; i += 64) {
+        if (i < SAVE_LONG) *colloid_word(d, g, i) = w[i];
+        else *colloid_int(d, g, i - SAVE_LONG) = (int)w[i];
+    }
+    if (g) return;
+    for (int r = threadIdx.x; r < ph.n_rep; r += 64) d.ev_total[r] = 0;
+    if (threadIdx.x == 0) {
+        *d.step -= 1;
+        *d.halt = 0;
+        d.status[1] = 0;
     }
 }
 
 // --------------------------------------------------------- colloid phases
 __global__ void k_colloid(Phys ph, Dev d, unsigned flags) {
+    if (stopped(ph, d)) return;
     int r = blockIdx.x;
     const Rep R = d.rep[r];
     colloid_phases(ph, d, R, r, flags);
@@ -153,6 +178,8 @@ __global__ __launch_bounds__(256) void k_tile_colloids(Phys ph, Dev d) {
         t0[a] = wrapi(tlo, R.nt[a]);
         nt[a] = min(thi - tlo + 1, R.nt[a]);
     }
+    if (stopped(ph, d)) return;
+    if (ph.groups) save_colloid(d, g, threadIdx.x, 256);
     for (int q = threadIdx.x; q < nt[0] * nt[1] * nt[2]; q += blockDim.x) {
         const int i = q % nt[0], j = (q / nt[0]) % nt[1], k = q / (nt[0] * nt[1]);
         const int tx = wrapi(t0[0] + i, R.nt[0]), ty = wrapi(t0[1] + j, R.nt[1]), tz = wrapi(t0[2] + k, R.nt[2]);
@@ -202,6 +229,7 @@ template <class Real>
 __global__ __launch_bounds__(DEPART_THREADS, 8) void k_depart(Phys ph, Dev d, Fluid<Real> f, const int2 *wgt, int nwg, int link) {
     static_assert(DEPART_THREADS == 256, "md_candidates: four waves");
     if ((int)blockIdx.x < nwg) {
+        if (stopped(ph, d)) return;
         md_candidates(ph, d, ld_const(wgt + blockIdx.x), link);
         return;
     }
@@ -219,6 +247,7 @@ __global__ __launch_bounds__(DEPART_THREADS, 8) void k_depart(Phys ph, Dev d, Fl
     // each wave owns a contiguous range of the tile's slots, in groups of 64
     const int per = ((n + NW - 1) / NW + 63) & ~63;
     const int lo = min(n, w * per), hi = min(n, lo + per);
+    if (stopped(ph, d)) return;
     for (int t = lane; t < 27; t += 64) s_cnt[w][t] = 0;
     if (w == NW - 1) {
         // the step's tile colloid lists, appended in arbitrary order, sorted:
@@ -494,6 +523,7 @@ __global__ __launch_bounds__(TH) void k_srd(Phys ph, Dev d, Fluid<Real> src, Flu
         zero_axis_masks(s_am[0]);
         if (NEAR_TEST) zero_axis_masks(s_am[1]);
     }
+    if (stopped(ph, d)) return;
     // gather offsets: an exclusive scan of the 27 list lengths across the
     // lanes of the first wave (the lists in direction order)
     if (threadIdx.x < 64) {
@@ -1514,7 +1544,7 @@ __global__ __launch_bounds__(256) void k_classify(Phys ph, Dev d, Fluid<Real> f)
     TileColl &tc = s_tc[w];
     NearColl &nf = s_nf[w];
     const unsigned long long below = (1ull << lane) - 1ull;
-    const int nchunk = ld_const(d.chunk_cnt);
+    const int nchunk = stopped(ph, d) ? 0 : ld_const(d.chunk_cnt);
     const int stride = gridDim.x * 4;
     bool drift = false;
     int ch = blockIdx.x * 4 + w;
@@ -1627,7 +1657,7 @@ __global__ __launch_bounds__(COLLIDE_THREADS) void k_collide(Phys ph, Dev d, Flu
 template <class Real>
 __global__ __launch_bounds__(COLLIDE_THREADS) void k_serial(Phys ph, Dev d, Fluid<Real> f, int substep) {
     __shared__ SerialLds s;
-    serial_replay<Real>(ph, d, f, substep, blockIdx.x, true, s);
+    serial_replay<Real>(ph, d, f, substep, blockIdx.x, s);
 }
 __global__ __launch_bounds__(256) void k_colloid_update(Phys ph, Dev d, unsigned flags, const int2 *wgt) {
     __shared__ UpdateLds s[4];
@@ -2116,7 +2146,7 @@ __global__ void k_gather(Phys ph, Dev d, Fluid<Real> f, double *pos, double *vel
 // 0..3 again); one thread per colloid was 84 us for 1227 colloids, this 8.7 us.
 __global__ __launch_bounds__(256) void k_features(Phys ph, Dev d, const int *colloid_rep) {
     const int g = blockIdx.x * (256 / 32) + threadIdx.x / 32, o = threadIdx.x % 32;
-    if (g >= ph.n_colloid_total) return;
+    if (g >= ph.n_colloid_total || stopped(ph, d)) return;
     const int r = colloid_rep[g];
     const Rep R = d.rep[r];
     const int L = R.L, Lc = L / 2;
@@ -2167,7 +2197,7 @@ __global__ __launch_bounds__(256) void k_features(Phys ph, Dev d, const int *col
 // clamped to the training range of the impulses, applied in n_sub equal parts
 __global__ void k_sur_sample(Phys ph, Dev d, const int *colloid_rep) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ph.n_colloid_total) return;
+    if (g >= ph.n_colloid_total || stopped(ph, d)) return;
     const Rep R = d.rep[colloid_rep[g]];
     const long long step = *d.step + 1;
     const uint32_t jl = (uint32_t)(g - R.first_colloid);
@@ -2202,6 +2232,7 @@ __global__ void k_sur_sample(Phys ph, Dev d, const int *colloid_rep) {
 template <class Real>
 __global__ __launch_bounds__(256) void k_sur_shell_kick(Phys ph, Dev d, Fluid<Real> f) {
     __shared__ double s_k[TCL_CAP][9];  // position, u, alpha
+    if (stopped(ph, d)) return;
     const int T = blockIdx.x;
     const int ns = min(d.tsl_cnt[T], TCL_CAP);
     if (ns == 0) return;
@@ -2468,6 +2499,9 @@ void launch_gather(const Phys &ph, const Dev &d, const Fluid<Real> &f, double *p
 }
 void launch_step_begin(const Phys &ph, const Dev &d, hipStream_t st, bool clear_lists) {
     LAUNCH(k_step_begin, clear_lists ? std::max(1, (ph.n_tiles + 255) / 256) : 1, 256, 0, st, ph, d, (int)clear_lists);
+}
+void launch_restore(const Phys &ph, const Dev &d, hipStream_t st) {
+    LAUNCH(k_restore, ph.n_colloid_total, 64, 0, st, ph, d);
 }
 void launch_colloid(const Phys &ph, const Dev &d, unsigned flags, hipStream_t st) {
     LAUNCH(k_colloid, ph.n_rep, 256, 0, st, ph, d, flags);

@@ -323,6 +323,11 @@ BW_API int bw_get_surrogate_shells(bw_ctx *ctx, int replica, int *count, double 
  * the last fused step's per-substep kernels touched ("near" a colloid under
  * blocked streaming; all particles under per-substep streaming). */
 BW_API int bw_near_particles(bw_ctx *ctx, int replica, long long *n_near);
+/* Fused steps since the context was created, by the way their substeps were
+ * taken (the results do not depend on it): by colloid groups, by groups first
+ * and kernel by kernel again (a cluster of colloids beyond a group's lists), and
+ * kernel by kernel at once. */
+BW_API int bw_step_paths(bw_ctx *ctx, long long *out3);
 
 #ifdef __cplusplus
 }

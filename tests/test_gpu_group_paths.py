@@ -78,3 +78,71 @@ def test_chain_across_half_the_box():
         v[:3] = [0, 23.0, 0]
 
     both(lambda s: place(s, np.array([[2.0 + 9 * i, 26, 26] for i in range(4)]), edit=edit), (1,), L=L, n_colloid=4)
+
+
+def sheet(k, n=None):
+    """k x k colloids that touch almost (linked into one group)"""
+    g = np.stack(np.meshgrid(np.arange(k), np.arange(k), indexing="ij"), -1).reshape(-1, 2)[:n]
+    return np.concatenate([3.0 + 5.0 * g, np.full((len(g), 1), 10.0)], 1)
+
+
+def lattice(n, spacing, origin=(2.0, 2.0, 2.0)):
+    k = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(k)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    return np.asarray(origin) + spacing * g
+
+
+def test_cluster_beyond_a_group():
+    """100 colloids in one cluster: such a step is taken kernel by kernel, and
+    soon only a few are tried by groups first (the tries 1, 3, 7, 15, ...)."""
+    a = both(lambda s: place(s, sheet(10)), (3, 12, 5), L=64, n_colloid=100)
+    assert a.step_paths() == dict(groups=0, again=4, per_substep=16)
+
+
+def test_groups_come_back():
+    """a cluster, then the same colloids far apart: steps by groups again"""
+    far = lattice(36, 13.0)
+
+    def prepare(s):
+        place(s, sheet(6))
+        s.step(4)
+        place(s, far)
+
+    a = both(prepare, (30, 10), L=52, n_colloid=36)
+    p = a.step_paths()
+    assert p["again"] == 2 and p["per_substep"] <= 5 and p["groups"] >= 37
+
+
+def test_a_new_start_forgets_clusters():
+    s = B.System(**BASE, L=40, n_colloid=36)
+    for n in (20, 0):
+        s.startup()
+        place(s, sheet(6))
+        s.step(n)
+    p = s.step_paths()
+    s.startup()
+    place(s, lattice(36, 10.0))
+    s.step(5)
+    q = s.step_paths()
+    assert q["groups"] == p["groups"] + 5 and q["again"] == p["again"] and q["per_substep"] == p["per_substep"]
+
+
+CROWDED = {
+    # events of a substep: about 240 against a list of 128
+    "events": (dict(L=40, n_colloid=24, n_sub=1, density=5), lambda: lattice(24, 5.0)),
+    # two colloids almost in one place (no forces): their particles are met by both, about 120 against a list of 16
+    "shared": (dict(L=40, n_colloid=24, n_sub=1, density=5, eps=0.0),
+               lambda: np.concatenate([lattice(12, 5.0), lattice(12, 5.0) + 0.2])),
+}
+
+
+@pytest.mark.parametrize("case", list(CROWDED))
+def test_lists_of_a_group_full(case):
+    prm, pos = CROWDED[case]
+    p = both(lambda s: place(s, pos()), (1,), **prm).step_paths()
+    assert p == dict(groups=0, again=1, per_substep=0)
+
+
+def test_small_groups_stay_by_groups():
+    p = both(lambda s: place(s, sheet(5, 24)), (2, 3), L=40, n_colloid=24).step_paths()
+    assert p == dict(groups=5, again=0, per_substep=0)
