@@ -625,8 +625,7 @@ int setup_groups(bw_ctx *c) {
         (rc = dalloc(c, &d.grp_hot, NC)) || (rc = dalloc(c, &d.grp_slot, NH)) ||
         (rc = dalloc(c, &d.grp_mem, NC)) || (rc = dalloc(c, &d.grp_big, NC)) || (rc = dalloc(c, &d.grp_small, NC)) ||
         (rc = dalloc(c, &d.grp_cnt, 2)) || (rc = dalloc(c, &d.hot_cnt, NC)) ||
-        (rc = dalloc(c, &d.hot_ent, NH)) || (rc = dalloc(c, &d.ovl_cnt, 1)) || (rc = dalloc(c, &d.ovl_g, OVL_CAP)) ||
-        (rc = dalloc(c, &d.ovl_slot, OVL_CAP)) || (rc = dalloc(c, &d.halt, 1)) || (rc = dalloc(c, &d.save, SAVE_WORDS * NC)))
+        (rc = dalloc(c, &d.hot_ent, NH)) || (rc = dalloc(c, &d.halt, 1)) || (rc = dalloc(c, &d.save, SAVE_WORDS * NC)))
         return rc;
     if ((rc = c->fp64 ? dalloc(c, &c->hot64, NH) : dalloc(c, &c->hot32, NH))) return rc;
     HIPCHK(c, hipHostMalloc((void **)&c->halt_step, sizeof(long long), hipHostMallocMapped));

@@ -49,7 +49,6 @@ constexpr int GROUP_MAX = 24;       // colloids of a group that a workgroup of i
 constexpr int GROUP_WIDE = 512;
 constexpr int GROUP_LDS_COLLOIDS = 3072;  // colloids that k_group_lists holds in LDS
 constexpr int SAVE_WORDS = 47;  // state of a colloid that a step by groups changes in place
-constexpr int OVL_CAP = 65536;      // hot particles beyond a full bucket, all colloids
 constexpr long long MEAN_CHUNK = 65536;  // particles per workgroup of the start-up's mean
 // workgroups per replica of the start-up's mean for replicas of up to max_nf particles
 inline int init_mean_chunks(long long max_nf) { return (int)std::max(1LL, (max_nf + MEAN_CHUNK - 1) / MEAN_CHUNK); }
@@ -170,9 +169,8 @@ struct Dev {
     int *grp_slot;       // the working copies' slots
     int2 *grp_big, *grp_small;  // groups of more than / up to GROUP_SMALL colloids: first member, size
     int *grp_cnt;        // their numbers
-    int *hot_cnt, *hot_ent;  // per colloid: slots of the particles that may reach it in the step
+    int *hot_cnt, *hot_ent;  // per colloid: slots of the (first hot_cap) particles that may reach it in the step
     int hot_cap;
-    int *ovl_cnt, *ovl_g, *ovl_slot;  // entries beyond a full bucket
     // a step by groups that could not be finished so: nonzero until the host
     // has taken it again; the kernels of the steps after it return at once
     int *halt;

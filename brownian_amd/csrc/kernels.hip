@@ -63,7 +63,6 @@ __global__ void k_step_begin(Phys ph, Dev d, int clear_lists) {
         *d.step = s;
         *d.chunk_cnt = 0;
         if (ph.groups) {
-            *d.ovl_cnt = 0;
             // the last step by groups was not stopped: its flags count
             if (d.status[1]) atomicOr(d.status, d.status[1]);
             d.status[1] = 0;
@@ -1627,19 +1626,8 @@ __global__ __launch_bounds__(256) void k_classify(Phys ph, Dev d, Fluid<Real> f)
         int base = 0;
         if (lead == lane) base = atomicAdd(&d.hot_cnt[home], num);
         base = __shfl(base, lead < 0 ? 0 : lead);
-        if (home >= 0) {
-            if (base + rank < d.hot_cap) {
-                d.hot_ent[(size_t)home * d.hot_cap + base + rank] = slot;
-            } else {
-                const int q = atomicAdd(d.ovl_cnt, 1);
-                if (q < OVL_CAP) {
-                    d.ovl_g[q] = home;
-                    d.ovl_slot[q] = slot;
-                } else {
-                    atomicOr(d.status, BW_FLAG_LIST_OVERFLOW);
-                }
-            }
-        }
+        // (the count shows k_group_lists a bucket that is full)
+        if (home >= 0 && base + rank < d.hot_cap) d.hot_ent[(size_t)home * d.hot_cap + base + rank] = slot;
     }
     if (drift) atomicOr(d.status, BW_FLAG_DRIFT);
 }

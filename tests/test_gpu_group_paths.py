@@ -146,3 +146,14 @@ def test_lists_of_a_group_full(case):
 def test_small_groups_stay_by_groups():
     p = both(lambda s: place(s, sheet(5, 24)), (2, 3), L=40, n_colloid=24).step_paths()
     assert p == dict(groups=5, again=0, per_substep=0)
+
+
+def test_full_buckets():
+    """Fluid that drifts by two cells a step past heavy colloids: more than
+    65536 particles beyond the colloids' buckets."""
+    def prepare(s):
+        p, v, _ = s.download_fluid()
+        s.upload_fluid(p, v + np.array([20.0, 0, 0]))
+
+    p = both(prepare, (1, 1), L=48, n_colloid=100, mass_colloid=1e7).step_paths()
+    assert p["groups"] == 0 and p["again"] >= 1
