@@ -9,8 +9,9 @@
 // (streaming, stochastic reflection in the reference's event order, serial
 // replay, WCA forces, Verlet, activity), with the colloids in LDS, in place of
 // four launches per substep over all of them.  A step that has a group of more
-// colloids or events than these lists hold is stopped (stop_step) and taken
-// again kernel by kernel.  The launches are bound by latency: 28 us a substep
+// colloids or events than these lists hold, or a reflected particle so fast that
+// it may come to another group, is stopped (stop_step) and taken again kernel by
+// kernel.  The launches are bound by latency: 28 us a substep
 // with 8 colloids (20^3), 35 with 300 (64^3), 54 with 2400 (128^3), of which
 // the kernels' first loads are most.  20 substeps by groups, with the
 // classification and the lists, take 0.19, 0.25 and 0.39 ms in place of 0.56,
@@ -69,21 +70,6 @@ struct GroupLds {
     int cnt[2][7];
 };
 
-// A particle at (x, y, z) after substep l, with speed v: may it come to an
-// explicitly colliding colloid that member(g) denies in the rest of the step?
-// From the colloids' positions at the step's start and their displacement bound.
-template <class F>
-__device__ inline bool reaches_other(const Phys &ph, const Dev &d, const Rep &R, double x, double y, double z, double v,
-                                     int l, F &&member) {
-    const double reach = sqrt(ph.lim_coll) + v * ph.dt * (ph.n_sub - 1 - l) + ph.margin, L = (double)R.L;
-    for (int g = R.first_colloid; g < R.first_colloid + R.nc; g++) {
-        if (member(g) || (ph.surrogate && d.cmode[g])) continue;
-        const double ax = img1(d.cpos[3 * g] - x, L), ay = img1(d.cpos[3 * g + 1] - y, L), az = img1(d.cpos[3 * g + 2] - z, L);
-        if ((ax * ax + ay * ay) + az * az <= reach * reach) return true;
-    }
-    return false;
-}
-
 // ---- k_groups' rare paths, kept out of line: inlined, they take it from 155
 // to 224 VGPRs.  They read the kernel's arguments where the launch put them (a
 // reference to by-value arguments would copy all of them to scratch memory).
@@ -99,15 +85,25 @@ template <class Real>
 __device__ __forceinline__ const GroupArgs<Real> *group_args() {  // the kernel's only argument
     return (const GroupArgs<Real> *)__builtin_amdgcn_kernarg_segment_ptr();
 }
-// reaches_other for the group of members g[0..C) of replica r
+// A particle at (x, y, z) after substep l, with speed v, reflected by the group
+// of members m[0..C) of replica r: may it come to an explicitly colliding
+// colloid of another group in the rest of the step?  From the colloids'
+// positions at the step's start and their displacement bound.
 template <class Real>
 __device__ __noinline__ bool group_reaches_other(const GroupArgs<Real> *a, int r, double x, double y, double z, double v, int l,
-                                                 const int *g, int C) {
-    return reaches_other(a->ph, a->d, a->d.rep[r], x, y, z, v, l, [&](int id) {
-        for (int c = 0; c < C; c++)
-            if (g[c] == id) return true;
-        return false;
-    });
+                                                 const int *m, int C) {
+    const Phys &ph = a->ph;
+    const Dev &d = a->d;
+    const Rep R = d.rep[r];
+    const double reach = sqrt(ph.lim_coll) + v * ph.dt * (ph.n_sub - 1 - l) + ph.margin, L = (double)R.L;
+    for (int g = R.first_colloid; g < R.first_colloid + R.nc; g++) {
+        bool member = false;
+        for (int c = 0; c < C; c++) member = member || m[c] == g;
+        if (member || (ph.surrogate && d.cmode[g])) continue;
+        const double ax = img1(d.cpos[3 * g] - x, L), ay = img1(d.cpos[3 * g + 1] - y, L), az = img1(d.cpos[3 * g + 2] - z, L);
+        if ((ax * ax + ay * ay) + az * az <= reach * reach) return true;
+    }
+    return false;
 }
 // the same for the reflected particle at LDS place i, if it is fast
 template <class Real, int NW>
@@ -821,9 +817,10 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
         unpack_cell(pc, ix, iy, iz);
         if (outside_tile_reach(R, ph.cap, slot, ix, iy, iz)) drift = true;
     }
+    if (escaped) stop_step(d);  // (that group is on its way, or done)
     unsigned st = 0;
     if (drift) st |= BW_FLAG_DRIFT;
-    if (marg || escaped) st |= BW_FLAG_MARGIN;
+    if (marg) st |= BW_FLAG_MARGIN;
     if (missing) st |= BW_FLAG_DRAW_MISSING;
     if (st) atomicOr(d.status, st);
     if (md_far) atomicOr(&d.md_stale[r], 1);

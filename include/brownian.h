@@ -43,9 +43,7 @@ extern "C" {
 #define BW_FLAG_ZERO_VARIANCE 0x80u    /* thermostat on a cell with zero relative KE      */
 #define BW_FLAG_NEIGH_OVERFLOW 0x100u  /* neigh_fl capacity exceeded                      */
 #define BW_FLAG_MARGIN 0x200u          /* a colloid moved beyond the blocked-streaming margin
-                                          within one step, or a reflected particle may have
-                                          reached one outside its group (use
-                                          BW_STREAM_PER_SUBSTEP)                         */
+                                          within one step (use BW_STREAM_PER_SUBSTEP)    */
 
 enum bw_precision { BW_FP32 = 0, BW_FP64 = 1 };
 enum bw_vel_law { BW_VEL_REFERENCE = 0, BW_VEL_MAXWELL = 1 };
@@ -325,8 +323,8 @@ BW_API int bw_get_surrogate_shells(bw_ctx *ctx, int replica, int *count, double 
 BW_API int bw_near_particles(bw_ctx *ctx, int replica, long long *n_near);
 /* Fused steps since the context was created, by the way their substeps were
  * taken (the results do not depend on it): by colloid groups, by groups first
- * and kernel by kernel again (a cluster of colloids beyond a group's lists), and
- * kernel by kernel at once. */
+ * and kernel by kernel again (a cluster of colloids beyond a group's lists, a
+ * reflected particle that may reach another group), and kernel by kernel at once. */
 BW_API int bw_step_paths(bw_ctx *ctx, long long *out3);
 
 #ifdef __cplusplus

@@ -157,3 +157,25 @@ def test_full_buckets():
 
     p = both(prepare, (1, 1), L=48, n_colloid=100, mass_colloid=1e7).step_paths()
     assert p["groups"] == 0 and p["again"] >= 1
+
+
+def spinning(neighbours, twice=1):
+    """A colloid (twice: two of them almost in one place, no forces) that spins
+    fast between neighbours just beyond the linking distance: a particle that it
+    reflects may come to one of them."""
+    c, e = np.array([10.0, 10, 10]), 5.45
+    around = np.array([[1.0, 0, 0], [-1, 0, 0], [0, 1, 0], [0, -1, 0]])[:neighbours]
+    pos = np.concatenate([[c, c + [0, 0, 0.1]][:twice], c + e * around])
+    omega = np.zeros_like(pos)
+    omega[:twice, 2] = 9.0
+    return both(lambda s: place(s, pos, omega), (1,), L=20, n_colloid=len(pos), density=20, mass_colloid=1e4,
+                eps=1.0 if twice == 1 else 0.0)
+
+
+@pytest.mark.parametrize("twice", [1, 2])
+def test_reflected_particle_that_may_reach_another_group(twice):
+    assert spinning(4, twice).step_paths() == dict(groups=0, again=1, per_substep=0)
+
+
+def test_fast_reflected_particle_alone():
+    assert spinning(0).step_paths() == dict(groups=1, again=0, per_substep=0)
