@@ -159,7 +159,7 @@ def test_full_buckets():
     assert p["groups"] == 0 and p["again"] >= 1
 
 
-def spinning(neighbours, twice=1):
+def spinning(neighbours, twice=1, steps=(1,), speed=9.0):
     """A colloid (twice: two of them almost in one place, no forces) that spins
     fast between neighbours just beyond the linking distance: a particle that it
     reflects may come to one of them."""
@@ -167,8 +167,8 @@ def spinning(neighbours, twice=1):
     around = np.array([[1.0, 0, 0], [-1, 0, 0], [0, 1, 0], [0, -1, 0]])[:neighbours]
     pos = np.concatenate([[c, c + [0, 0, 0.1]][:twice], c + e * around])
     omega = np.zeros_like(pos)
-    omega[:twice, 2] = 9.0
-    return both(lambda s: place(s, pos, omega), (1,), L=20, n_colloid=len(pos), density=20, mass_colloid=1e4,
+    omega[:twice, 2] = speed
+    return both(lambda s: place(s, pos, omega), steps, L=20, n_colloid=len(pos), density=20, mass_colloid=1e4,
                 eps=1.0 if twice == 1 else 0.0)
 
 
@@ -179,3 +179,118 @@ def test_reflected_particle_that_may_reach_another_group(twice):
 
 def test_fast_reflected_particle_alone():
     assert spinning(0).step_paths() == dict(groups=1, again=0, per_substep=0)
+
+
+def test_stopped_steps_among_others():
+    """some of the steps of one call are stopped, with steps by groups before and behind them"""
+    p = spinning(4, steps=(1, 12, 1, 1, 6), speed=7.5).step_paths()
+    assert p["groups"] >= 4 and p["again"] >= 2 and sum(p.values()) == 21
+
+
+CLUSTER = dict(L=32, n_colloid=25, n_sub=4, density=5)  # beyond a group: every step is stopped
+
+
+@pytest.mark.parametrize("read", ["status", "audit", "observables", "md_list", "run_counts", "near_particles", "updown"])
+def test_reads_behind_a_stopped_step(read):
+    """the same as when the steps have been waited for"""
+    def result(wait):
+        s = B.System(**{**BASE, **CLUSTER})
+        s.startup()
+        place(s, sheet(5))
+        s.neighbour_list_mpcd()
+        s.observables_reset()
+        s.step(2)
+        if wait:
+            s.sync()
+        if read == "updown":
+            s.neighbour_list_mpcd()
+            s.updown_velocity()
+        r = getattr(s, read)()
+        assert s.step_paths()["again"] >= 1
+        return r if isinstance(r, dict) else dict(enumerate(r if isinstance(r, tuple) else (r,)))
+
+    a, b = result(False), result(True)
+    for k in a:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=str(k))
+
+
+@pytest.mark.parametrize("entry", ["set_v0", "upload_fluid", "upload_colloid", "rotation_mpcd", "run", "update_pos_md",
+                                   "update_pos_mpcd", "substep", "set_moments", "profile_steps", "time_steps"])
+def test_changes_behind_a_stopped_step(entry):
+    def change(s):
+        place(s, sheet(5))
+        s.step(2)
+        if entry == "set_v0":
+            s.set_v0(np.full(25, 0.3))
+        elif entry == "upload_fluid":
+            p, v, _ = s.download_fluid()
+            s.step(1)
+            s.upload_fluid(p, v)
+        elif entry == "upload_colloid":
+            s.upload_colloid(vel=np.full((25, 3), 0.1))
+        elif entry in ("profile_steps", "time_steps"):
+            getattr(s, entry)(3)
+        else:
+            getattr(s, entry)()
+
+    both(change, (2,), **CLUSTER)
+
+
+def test_injected_draws_in_a_stopped_step():
+    import oracle as O
+    from tests.parity import compare_state, inject_step, oracle_step_draws
+    prm = dict(L=30, density=5, n_colloid=25, sig_colloid=4.2, sigma=4.0, mass_colloid=50.0, n_sub=4, v0=0.01, theta_deg=90.0, seed=99)
+    s = B.System(precision=B.BW_FP64, draws=B.BW_DRAWS_INJECTED, **prm)
+    s.startup()
+    place(s, sheet(5))
+    o = O.Oracle(**prm)
+    o.startup()
+    o.set_fluid(*s.download_fluid()[:2])
+    o.set_colloid(**s.download_colloid())
+    o.neighbour_list_mpcd()
+    o.neighbour_list_md()
+    for _ in range(2):
+        shift, axes, refl = oracle_step_draws(o, prm["n_sub"])
+        inject_step(s, shift, axes, refl)
+        s.step(1)
+        assert s.status() == 0
+        compare_state(s, o, prm["L"], 1e-10, 1e-10, 1e-10)
+    assert s.step_paths()["again"] >= 1
+
+
+@pytest.mark.parametrize("colloids", [24, 25])
+def test_driven_and_explicit_colloids_in_one_group(colloids):
+    """The surrogate drives about half of a cluster's colloids: in one group (24), in a stopped step (25)."""
+    rng = np.random.default_rng(8)
+    net = B.MLP(1)
+    net.set_params((0.05 * rng.standard_normal(net.n_params)).astype(np.float32))
+    lo, hi = np.full(144, -1e30), np.full(144, 1e30)
+    lo[141] = 0.0  # those that point to +x
+
+    def attach(s):
+        place(s, sheet(5, colloids))
+        s.surrogate_attach(net, lo, hi, np.full(6, -20.0), np.full(6, 20.0))
+        s.step(1)  # the first has no moments yet: explicit
+
+    s = both(attach, (1, 3), L=32, n_colloid=colloids, n_sub=10, v0=0.03)
+    _, imp, mode = s.surrogate_data()
+    assert 0 < mode.sum() < colloids and np.abs(imp).sum() > 0
+    p = s.step_paths()
+    assert p["groups"] == 5 if colloids == 24 else p["again"] >= 2
+
+
+def test_more_colloids_than_the_lists_in_lds():
+    """k_group_lists beyond 3072 colloids"""
+    prm = [dict(BASE, density=5, L=16, n_colloid=8, n_sub=2, seed=100 + r) for r in range(400)]
+    a, b = (B.System(replicas=[dict(p, streaming=v) for p in prm]) for v in (B.BW_STREAM_BLOCKED, B.BW_STREAM_PER_SUBSTEP))
+    for s in (a, b):
+        s.startup()
+        s.step(2)
+        assert s.status() == 0
+    assert a.step_paths() == dict(groups=2, again=0, per_substep=0)
+    for r in range(0, 400, 57):
+        ca, cb = a.download_colloid(r), b.download_colloid(r)
+        for k in ca:
+            np.testing.assert_array_equal(ca[k], cb[k], err_msg=k)
+        for x, y in zip(a.download_fluid(r), b.download_fluid(r)):
+            np.testing.assert_array_equal(x, y)
