@@ -18,10 +18,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 #include "bw_common.h"
 
@@ -45,7 +44,7 @@ class Staging {
     Staging(const Staging &) = delete;
     Staging &operator=(const Staging &) = delete;
     ~Staging() {
-        for (hipEvent_t e : ev_) (void)hipEventDestroy(e);
+        for (int i = 0; i < n_ev_; i++) (void)hipEventDestroy(ev_[i]);
         if (buf_) (void)hipHostFree(buf_);
     }
 
@@ -71,7 +70,8 @@ class Staging {
     std::mutex m_;
     char *buf_ = nullptr;
     size_t cap_ = 0;
-    std::vector<hipEvent_t> ev_;
+    hipEvent_t ev_[2 * THREADS];
+    int n_ev_ = 0;
 
     bool reserve(size_t bytes, int events) {
         if (bytes > cap_) {
@@ -87,14 +87,11 @@ class Staging {
             buf_ = (char *)p;
             cap_ = bytes;
         }
-        while ((int)ev_.size() < events) {
-            hipEvent_t e;
-            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        for (; n_ev_ < events; n_ev_++)
+            if (hipEventCreateWithFlags(&ev_[n_ev_], hipEventDisableTiming) != hipSuccess) {
                 (void)hipGetLastError();
                 return false;
             }
-            ev_.push_back(e);
-        }
         return true;
     }
     // no pinned memory to be had
@@ -120,7 +117,8 @@ class Staging {
     }
     // The pieces are handed out in order.  A thread owns two places of the
     // buffer and their events: while one piece is copied out the next is on
-    // its way.  (A thread that cannot be started leaves its share to the others.)
+    // its way.  (A thread that cannot be started, for want of memory or of
+    // threads, leaves its share to the others.)
     hipError_t pieces(const StageSeg *s, int k, int nt, hipStream_t st) {
         size_t first[PackSegs::MAX + 1] = {0};
         for (int i = 0; i < k; i++) first[i + 1] = first[i] + (s[i].bytes + CHUNK - 1) / CHUNK;
@@ -156,14 +154,14 @@ class Staging {
             }
             if (e != hipSuccess) error.store((int)e);
         };
-        std::vector<std::thread> threads;
-        threads.reserve(nt);
+        std::thread threads[THREADS];
         try {
-            for (int w = 1; w < nt; w++) threads.emplace_back(work, w);
-        } catch (const std::system_error &) {
+            for (int w = 1; w < nt; w++) threads[w] = std::thread(work, w);
+        } catch (const std::exception &) {
         }
         work(0);
-        for (auto &t : threads) t.join();
+        for (auto &t : threads)
+            if (t.joinable()) t.join();
         const hipError_t e = hipStreamSynchronize(st);  // also after an error: nothing of the buffer is in flight
         return error.load() != hipSuccess ? (hipError_t)error.load() : e;
     }
