@@ -95,6 +95,8 @@ struct QueuedStep {
     bool final, prologue;
 };
 
+constexpr size_t MAX_QUEUED = 8192;
+
 struct FluidAlloc {
     void *base = nullptr;
     Fluid<float> f32;
@@ -148,7 +150,7 @@ struct bw_ctx {
     HotPart<float> *hot32 = nullptr;
     HotPart<double> *hot64 = nullptr;
     long long *halt_step = nullptr;
-    std::vector<QueuedStep> queued;
+    std::vector<QueuedStep> queued, again;  // MAX_QUEUED each, so that stepping allocates nothing
     // steps finished by groups since one was stopped; steps to take kernel by
     // kernel before the next try, and how many the last time; that try follows
     int good = 0, skip = 0, backoff = 0;
@@ -486,7 +488,7 @@ int one_step(bw_ctx *c, bool final, Prof *prof) {
 // idle: the stream has been waited for.
 template <class Real>
 int settle_impl(bw_ctx *c, bool idle) {
-    std::vector<QueuedStep> again;  // the first is next
+    std::vector<QueuedStep> &again = c->again;  // steps to take again, the first is next
     for (;;) {
         if (!c->queued.empty()) {
             if (!idle) HIPCHK(c, hipStreamSynchronize(c->st));
@@ -557,7 +559,7 @@ int do_steps(bw_ctx *c, int n, Prof *prof) {
         if ((rc = one_step<Real>(c, s == n - 1, prof))) return rc;
         // a try after stopped steps is looked at before more follow it; and
         // the list of steps stays bounded
-        if ((c->trying && !c->queued.empty()) || c->queued.size() >= 65536) {
+        if ((c->trying && !c->queued.empty()) || c->queued.size() >= MAX_QUEUED) {
             if ((rc = settle(c))) return rc;
         }
     }
@@ -630,6 +632,8 @@ int setup_groups(bw_ctx *c) {
     if ((rc = c->fp64 ? dalloc(c, &c->hot64, NH) : dalloc(c, &c->hot32, NH))) return rc;
     HIPCHK(c, hipHostMalloc((void **)&c->halt_step, sizeof(long long), hipHostMallocMapped));
     *c->halt_step = 0;
+    c->queued.reserve(MAX_QUEUED);
+    c->again.reserve(MAX_QUEUED);
     HIPCHK(c, hipHostGetDevicePointer((void **)&d.halt_step, c->halt_step, 0));
     c->groups = true;
     return BW_OK;
@@ -1115,6 +1119,7 @@ BW_API int initialize(bw_ctx *c) {
     HIPCHK(c, hipMemsetAsync(c->dv.status, 0, 2 * sizeof(unsigned), c->st));
     // of earlier steps nothing counts any more, also not that one was stopped
     c->queued.clear();
+    c->again.clear();
     c->good = c->skip = c->backoff = 0;
     c->trying = false;
     if (c->groups) {

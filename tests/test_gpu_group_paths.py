@@ -294,3 +294,18 @@ def test_more_colloids_than_the_lists_in_lds():
             np.testing.assert_array_equal(ca[k], cb[k], err_msg=k)
         for x, y in zip(a.download_fluid(r), b.download_fluid(r)):
             np.testing.assert_array_equal(x, y)
+
+
+def test_more_steps_than_the_list_of_launched_ones():
+    """8192 steps may be launched before they are looked at"""
+    a, b = (B.System(**{**BASE, "L": 8, "n_colloid": 1, "n_sub": 2, "density": 2, "streaming": v})
+            for v in (B.BW_STREAM_BLOCKED, B.BW_STREAM_PER_SUBSTEP))
+    for s in (a, b):
+        s.startup()
+        s.step(8200)
+        for _ in range(30):
+            s.step(1)
+        assert s.status() == 0
+    assert a.step_paths()["groups"] == 8230
+    for x, y in zip(state(a).values(), state(b).values()):
+        np.testing.assert_array_equal(x, y)
