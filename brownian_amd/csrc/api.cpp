@@ -622,19 +622,24 @@ int setup_groups(bw_ctx *c) {
     ph.window_min = std::max(1, ph.window / 3);
     // a colloid's events per substep must fit a group's list with room to spare
     if (density * area * 0.4 * ph.vscale_thermal * ph.dt > 12.0) return BW_OK;
-    int rc;
-    if ((rc = dalloc(c, &d.uf, NC)) || (rc = dalloc(c, &d.uf_linked, NC)) || (rc = dalloc(c, &d.grp_root, 4 * NC)) ||
-        (rc = dalloc(c, &d.grp_hot, NC)) || (rc = dalloc(c, &d.grp_slot, NH)) ||
-        (rc = dalloc(c, &d.grp_mem, NC)) || (rc = dalloc(c, &d.grp_big, NC)) || (rc = dalloc(c, &d.grp_small, NC)) ||
-        (rc = dalloc(c, &d.grp_cnt, 2)) || (rc = dalloc(c, &d.hot_cnt, NC)) ||
-        (rc = dalloc(c, &d.hot_ent, NH)) || (rc = dalloc(c, &d.halt, 1)) || (rc = dalloc(c, &d.save, SAVE_WORDS * NC)))
-        return rc;
-    if ((rc = c->fp64 ? dalloc(c, &c->hot64, NH) : dalloc(c, &c->hot32, NH))) return rc;
-    HIPCHK(c, hipHostMalloc((void **)&c->halt_step, sizeof(long long), hipHostMallocMapped));
+    const size_t held = c->allocs.size();
+    const bool short_of_memory =
+        dalloc(c, &d.uf, NC) || dalloc(c, &d.uf_linked, NC) || dalloc(c, &d.grp_root, 4 * NC) || dalloc(c, &d.grp_hot, NC) ||
+        dalloc(c, &d.grp_slot, NH) || dalloc(c, &d.grp_mem, NC) || dalloc(c, &d.grp_big, NC) || dalloc(c, &d.grp_small, NC) ||
+        dalloc(c, &d.grp_cnt, 2) || dalloc(c, &d.hot_cnt, NC) || dalloc(c, &d.hot_ent, NH) || dalloc(c, &d.halt, 1) ||
+        dalloc(c, &d.save, SAVE_WORDS * NC) || (c->fp64 ? dalloc(c, &c->hot64, NH) : dalloc(c, &c->hot32, NH)) ||
+        hipHostMalloc((void **)&c->halt_step, sizeof(long long), hipHostMallocMapped) != hipSuccess;
+    if (short_of_memory) {  // a context that just fits steps kernel by kernel
+        (void)hipGetLastError();
+        for (; c->allocs.size() > held; c->allocs.pop_back()) hipFree(c->allocs.back());
+        c->halt_step = nullptr;
+        c->err.clear();
+        return BW_OK;
+    }
     *c->halt_step = 0;
+    HIPCHK(c, hipHostGetDevicePointer((void **)&d.halt_step, c->halt_step, 0));
     c->queued.reserve(MAX_QUEUED);
     c->again.reserve(MAX_QUEUED);
-    HIPCHK(c, hipHostGetDevicePointer((void **)&d.halt_step, c->halt_step, 0));
     c->groups = true;
     return BW_OK;
 }
