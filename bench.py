@@ -35,6 +35,7 @@ import csv
 import glob
 import json
 import os
+import re
 import sys
 import time
 
@@ -52,7 +53,7 @@ COPY_BYTES = 1 << 30     # calibration copy: reads and writes this many bytes
 #   stream  read cell+offsets 16 + velocities 12, write cell+offsets 16 (near particles)
 #   depart  read cell+offsets 16, write the departure index 4
 ALG_BYTES = {"srd": 64, "stream": 44, "depart": 20}
-PMC_FILE = os.path.join(ROOT, "profiles", "srd_kernel_128cubed_pmc.json")
+PMC_FILES = os.path.join(ROOT, "profiles", "srd_kernel_128cubed_pmc*.json")  # one per tile shape
 
 
 def log(msg):
@@ -155,7 +156,7 @@ def _per_kernel(rows, counter):
             continue
         name = r.get("Kernel_Name", "")
         base = next((k for k in ("k_srd", "k_stream", "k_depart", "k_collide", "k_colloid_update", "k_copy",
-                                 "k_md_candidates", "k_tile_colloids") if k in name), None)
+                                 "k_classify", "k_groups", "k_tile_colloids") if k in name), None)
         if base is None:
             continue
         key = (base, r.get("Dispatch_Id") or r.get("Correlation_Id"))
@@ -184,6 +185,17 @@ def pmc_summary(fetch_dir, write_dir, out_file, command):
     with open(out_file, "w") as fh:
         json.dump(res, fh, indent=1)
     print(json.dumps(res, indent=1))
+
+
+def srd_traffic(tile):
+    """k_srd's counted bytes per launch with this tile shape (None: not counted)"""
+    for f in sorted(glob.glob(PMC_FILES)):
+        with open(f) as fh:
+            d = json.load(fh)
+        m = re.search(r"--tile (\d+) (\d+) (\d+)", d["command"])
+        if m and [int(b) for b in m.groups()] == list(tile):
+            return d["kernels"]["k_srd"]["bytes_per_launch"]
+    return None
 
 
 # ---------------------------------------------------------------- ensemble
@@ -399,12 +411,7 @@ def main():
         kern[k] = e
     dom = max(kern, key=lambda k: kern[k]["ms_per_step"])
     rk = "srd"  # the HBM kernel that moves every particle of the blocked step
-    traffic = None
-    if os.path.exists(PMC_FILE):
-        try:
-            traffic = json.load(open(PMC_FILE))["kernels"]["k_srd"]["bytes_per_launch"]
-        except Exception:
-            traffic = None
+    traffic = srd_traffic(tile_used) if (args.L, args.ncol) == (128, 2400) else None
     copy_ms = s.debug_copy_ms(COPY_BYTES, reps=args.copy_reps)
     copy_bw = 2 * COPY_BYTES / (copy_ms / 1e3)
 
