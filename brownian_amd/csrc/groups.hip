@@ -26,8 +26,8 @@ namespace bw {
 constexpr int CURRENT = (int)(1u << 31);
 constexpr int IN_WINDOW = -1;
 
-// What a group of NW waves holds: a wave takes one or two colloids (most
-// groups), a workgroup of four waves more.
+// What a group of NW waves holds: a wave takes a lone colloid, a workgroup of
+// four waves 2 to GROUP_MAX (or every group, up to GROUP_WIDE colloids in all).
 template <int NW>
 struct GroupCaps {
     static constexpr int MAX = NW == 1 ? GROUP_SMALL : GROUP_MAX;  // colloids

@@ -377,7 +377,10 @@ struct bw_mlp {
     long long adam_t = 0;
     MlpBuf tb;  // training / host-call activations
     unsigned char *scratch = nullptr;  // device address of the scratch array on the network's GPU
-    float *xin = nullptr, *tin = nullptr, *yout = nullptr;  // a host call's rows (grown as needed)
+    // a host call's rows: 648 bytes for each of the largest call's, kept until
+    // the network is destroyed, as its activations are (two hipMalloc and hipFree
+    // a call otherwise)
+    float *xin = nullptr, *tin = nullptr, *yout = nullptr;
     float *ypin = nullptr;    // outputs of up to PINNED_ROWS rows, in pinned host memory
     long long xin_rows = 0;
     // data set on the device, and the rows' losses
@@ -750,16 +753,17 @@ BW_API int bw_mlp_loss_grad(bw_mlp *m, const float *x, const float *t, int n, do
     if (!m || !x || !t || n < 1) return BW_ERR_ARG;
     int n_pad = (n + 31) / 32 * 32, rc;
     if ((rc = ensure_batch(m, n_pad, true)) || (rc = ensure_rows(m, n))) return rc;
+    // (queued, unlike bw_mlp_forward's: two copies and many launches follow, and
+    // the waits of plain ones cost more than the slower copies: 20 rows 164
+    // against 179 us)
     MCHK(m, hipMemcpyAsync(m->xin, x, sizeof(float) * (size_t)n * MLP_IN, hipMemcpyHostToDevice, m->st));
     MCHK(m, hipMemcpyAsync(m->tin, t, sizeof(float) * (size_t)n * MLP_T, hipMemcpyHostToDevice, m->st));
     const ParamTable tab = loss_backward(m, m->tb, m->xin, m->tin, nullptr, n, n_pad, m->tb.loss, m->st);
     std::vector<float> l(loss ? n : 0);
     if (loss) MCHK(m, hipMemcpyAsync(l.data(), m->tb.loss, sizeof(float) * n, hipMemcpyDeviceToHost, m->st));
-    if (grad) {
-        if ((rc = copy_params(m, grad, tab, true))) return rc;
-    } else {
-        MCHK(m, hipStreamSynchronize(m->st));
-    }
+    rc = grad ? copy_params(m, grad, tab, true) : BW_OK;
+    MCHK(m, hipStreamSynchronize(m->st));  // also after an error: l is a copy's destination
+    if (rc) return rc;
     if (loss) {
         double s = 0;
         for (int i = 0; i < n; i++) s += l[i];

@@ -293,7 +293,7 @@ BW_API int bw_mlp_train(bw_mlp *m, const float *x, const float *t, int n, int ep
  * raw features) and y (n x 12, the bw_mlp_forward outputs) are DEVICE
  * pointers on the network's GPU; the activations live in a fixed device
  * array of the library (at most 1024 rows; larger n is BW_ERR_ARG, about
- * 7.9 MiB held by each GPU until the process ends), so the call allocates
+ * 1.9 MiB held by each GPU until the process ends), so the call allocates
  * nothing.  It synchronises the network's stream before returning.  Calls
  * that overlap on one GPU share that array and race. */
 BW_API int bw_mlp_forward_noalloc(bw_mlp *m, const float *x, int n, float *y);
