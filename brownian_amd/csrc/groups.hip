@@ -11,11 +11,10 @@
 // four launches per substep over all of them.  A step that has a group of more
 // colloids or events than these lists hold, or a reflected particle so fast that
 // it may come to another group, is stopped (stop_step) and taken again kernel by
-// kernel.  The launches are bound by latency: 28 us a substep
-// with 8 colloids (20^3), 35 with 300 (64^3), 54 with 2400 (128^3), of which
-// the kernels' first loads are most.  20 substeps by groups, with the
-// classification and the lists, take 0.19, 0.25 and 0.39 ms in place of 0.56,
-// 0.69 and 1.06 (FP32; FP64 at 20^3).
+// kernel.  Those launches are bound by latency: 28 us a substep with 8 colloids
+// (20^3), 35 with 300 (64^3), 54 with 2400 (128^3), of which the kernels' first
+// loads are most.  20 substeps by groups, with the classification and the lists,
+// take 0.14, 0.17 and 0.31 ms in place of 0.56, 0.69 and 1.06 (FP32; FP64 at 20^3).
 #include "bw_device.h"
 #include "collide.h"
 
@@ -379,7 +378,8 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
         const float4 b = s.rel[0][c];
         extent = fmaxf(extent, fmaxf(fabsf(b.x), fmaxf(fabsf(b.y), fabsf(b.z))));
     }
-    const float room = 0.5f * Lf - 1.0f - (extent + (float)ph.margin + 1e-2f);
+    const float room = __int_as_float(__builtin_amdgcn_readfirstlane(  // the same in every lane
+        __float_as_int(0.5f * Lf - 1.0f - (extent + (float)ph.margin + 1e-2f))));
     unsigned all = 0;  // the explicitly colliding colloids
     for (int c = 0; c < C; c++)
         if (!s.sur[c]) all |= 1u << c;
@@ -887,9 +887,10 @@ __global__ __launch_bounds__(1024) void k_group_lists(Phys ph, Dev d) {
 
 // One workgroup per large group, then one wave per small one; WIDE: a workgroup
 // for every group (up to GROUP_WIDE colloids).  Two workgroups per CU are all
-// that a WIDE launch has (226 VGPRs, none spilled); the other takes three in
-// FP32 (168, some spilled), which 2400 groups need to run at once.  final: the
-// last substep ends with update_velocity_colloid (no kick, no position update).
+// that a WIDE launch has (212 VGPRs, none spilled; 252 and some in FP64); the
+// other takes three in FP32 (168, some spilled), which 2400 groups need to run
+// at once.  final: the last substep ends with update_velocity_colloid (no kick,
+// no position update).
 template <class Real, bool WIDE>
 __global__ __launch_bounds__(256, WIDE || sizeof(Real) == 8 ? 2 : 3) void k_groups(GroupArgs<Real> a) {
     const Phys &ph = a.ph;

@@ -8,7 +8,9 @@
  * cpp/active_brownian.cpp:3-7).  Here each keeps its name, takes the context
  * that owns that state and returns a status code (BW_OK or a negative BW_ERR_*).
  * Calls are asynchronous on the context's HIP stream; calls that return data to
- * the host synchronise.  One context per host thread.
+ * the host synchronise.  Steps count as taken when the next call on the context
+ * returns (bw_sync at the latest), not when the stream has run empty: a step
+ * may have to be taken again (bw_step_paths).  One context per host thread.
  *
  * Units and indices: box edge L cells of size a = 1; particle, colloid and cell
  * indices are 0-based (the reference is 1-based); positions, velocities and
