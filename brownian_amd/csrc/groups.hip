@@ -654,6 +654,11 @@ __device__ __forceinline__ bool group_step(const Phys &ph, const Dev &d, const F
         sync();
         const int n_cont = cnt[2];
         if (n_cont > G::SER) return false;
+        // more events of a colloid than the per-substep kernels' bucket holds:
+        // those are replayed serially there, by id (fluid inside a colloid)
+        if (G::EV > EV_CAP && n_ev > EV_CAP)
+            for (int c = 0; c < C; c++)
+                if (s.nev[c] > EV_CAP) return false;
         if (cnt[6])
             for (int e = tid; e < n_ev; e += TH)
                 if (fast_event<Real, NW>(group_args<Real>(), r, l, C, s.ev_i[e], &s)) escaped = true;

@@ -143,6 +143,19 @@ def test_lists_of_a_group_full(case):
     assert p == dict(groups=0, again=1, per_substep=0)
 
 
+def test_more_events_of_a_colloid_than_its_bucket():
+    """Fluid inside a colloid, 64 to 128 events of it in a substep: the
+    per-substep kernels replay them serially, in another order of the sums."""
+    pos = np.array([[8.3, 8.1, 7.9]])
+
+    def put(s):
+        z = np.zeros_like(pos)
+        s.upload_colloid(pos=pos, vel=z, omega=z, f=z, old_f=z)
+
+    p = both(put, (1, 2), L=16, n_colloid=1, density=3, mass_colloid=654.1).step_paths()
+    assert p["again"] >= 1
+
+
 def test_small_groups_stay_by_groups():
     p = both(lambda s: place(s, sheet(5, 24)), (2, 3), L=40, n_colloid=24).step_paths()
     assert p == dict(groups=5, again=0, per_substep=0)
