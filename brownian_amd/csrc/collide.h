@@ -394,13 +394,18 @@ __device__ __forceinline__ void colloid_update_wave(const Phys &ph, const Dev &d
     }
     // lanes 0-5: sin (lanes 0-2) or cos (lanes 3-5) of the activity rotation
     // angle about axis lane % 3, from the angular velocity after the impulse,
-    // formed as colloid_update forms them; lane 0 gathers them below
+    // formed as colloid_update forms them (a surrogate-driven colloid's torque
+    // may be the mirrored fluid's); lane 0 gathers them below
+    const bool driven = (flags & PH_APPLY) && ph.surrogate && d.cmode[gs];
+    double torque[3] = {0, 0, 0};
+    if (driven)
+        for (int k = 0; k < 3; k++) torque[k] = __shfl(lane == 0 ? in.sv[3 + k] : 0.0, 0);
     double tv = 0.0;
     if ((flags & PH_ACTIVITY) && lane < 6) {
         const int k = lane % 3;
         double wk = d.comega[3 * gs + k];
         if (flags & PH_APPLY) {
-            const double iw = (ph.surrogate && d.cmode[gs]) ? d.csur[6 * gs + 3 + k] : d.cdw[3 * gs + k];
+            const double iw = driven ? (k == 0 ? torque[0] : k == 1 ? torque[1] : torque[2]) : d.cdw[3 * gs + k];
             wk = wk + iw * ph.mass_fl / ph.I_colloid;
         }
         const double b = wk * ph.dt;

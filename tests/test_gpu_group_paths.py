@@ -271,25 +271,38 @@ def test_injected_draws_in_a_stopped_step():
     assert s.step_paths()["again"] >= 1
 
 
-@pytest.mark.parametrize("colloids", [24, 25])
-def test_driven_and_explicit_colloids_in_one_group(colloids):
-    """The surrogate drives about half of a cluster's colloids: in one group (24), in a stopped step (25)."""
+def attach_random_network(s, driven=0.0):
+    """drives the colloids whose orientation's x is above `driven`, from the second step on"""
     rng = np.random.default_rng(8)
     net = B.MLP(1)
     net.set_params((0.05 * rng.standard_normal(net.n_params)).astype(np.float32))
     lo, hi = np.full(144, -1e30), np.full(144, 1e30)
-    lo[141] = 0.0  # those that point to +x
+    lo[141] = driven
+    s.surrogate_attach(net, lo, hi, np.full(6, -20.0), np.full(6, 20.0))
+    s.step(1)
 
+
+@pytest.mark.parametrize("colloids", [24, 25])
+def test_driven_and_explicit_colloids_in_one_group(colloids):
+    """The surrogate drives about half of a cluster's colloids: in one group (24), in a stopped step (25)."""
     def attach(s):
         place(s, sheet(5, colloids))
-        s.surrogate_attach(net, lo, hi, np.full(6, -20.0), np.full(6, 20.0))
-        s.step(1)  # the first has no moments yet: explicit
+        attach_random_network(s)
 
     s = both(attach, (1, 3), L=32, n_colloid=colloids, n_sub=10, v0=0.03)
     _, imp, mode = s.surrogate_data()
     assert 0 < mode.sum() < colloids and np.abs(imp).sum() > 0
     p = s.step_paths()
     assert p["groups"] == 5 if colloids == 24 else p["again"] >= 2
+
+
+def test_driven_colloids_with_thin_shells():
+    """Shells of about 19 particles: some are too thin for the torque (fewer than
+    16), some for the impulse (8), and the colloid takes the mirrored fluid's back."""
+    s = both(lambda s: attach_random_network(s, -2.0), (1, 5, 2), L=24, n_colloid=40, n_sub=6, density=1, v0=0.2, sigma=3.0,
+             sig_colloid=3.15)
+    count, _ = s.surrogate_shells()
+    assert (count < 16).any() and s.step_paths()["groups"] == 9
 
 
 def test_more_colloids_than_the_lists_in_lds():
